@@ -443,6 +443,54 @@ int spira_hip_conv_ws_fused(int64_t num_sources, int64_t num_targets, const int3
                             int c_in, const void *weights, const void *prepared, int num_weights, int c_out,
                             int dtype, float *target_acc, hipStream_t stream);
 
+/* Fragment-major copy of weights [K, c_in, c_out] for spira_hip_conv_map,
+ * conv_masks and conv_pairs: per offset, 16-column tile and 64 bytes of input
+ * channels, one 1 KB block in the lane order of the matrix instructions,
+ * zero-padded.  Valid until the weights change.  (No reference counterpart.) */
+int spira_hip_fragments_bytes(int num_offsets, int c_in, int c_out, int dtype, size_t *bytes);
+int spira_hip_prepare_fragments(const void *weights, int num_offsets, int c_in, int c_out, int dtype, void *fragments,
+                                hipStream_t stream);
+
+/* rows [num_sources, row_channels] = sources [num_sources, c_in], zero past
+ * c_in: the source rows the compacted convolutions gather when c_in is not a
+ * multiple of 16 bytes.  (No reference counterpart.) */
+int spira_hip_pad_rows(const void *sources, int64_t num_sources, int c_in, int row_channels, int dtype, void *rows,
+                       hipStream_t stream);
+
+/* Sparse convolution over the valid (source, target) pairs, compacted block
+ * by block: targets[t] = epilogue(sum_k sources[s(t, k)] @ weights[k]), fp32
+ * sums in offset order, the epilogue of spira_hip_conv_os.  Source rows hold
+ * row_channels values: c_in rounded up to 16 bytes (the added ones unused,
+ * any finite value); sources start on a 16-byte boundary.  conv_map takes a
+ * map [>= num_targets, num_offsets]; conv_masks the ranks of
+ * spira_hip_kmap_emit_masks ([num_offsets, S] and [num_offsets, T]);
+ * conv_pairs compacted rows of pairs as spira_hip_conv_ws_fused takes them
+ * (mirror_rows too; pairs in any order).  The last two run a hybrid's dense
+ * offsets first when dense_offsets > 0: dense_map [>= num_targets,
+ * dense_offsets], or null for one identity offset; the weights then hold the
+ * dense rows first.  Their workspace is scratch (no initial contents);
+ * nothing is read back on the host.  (reference: the same dataflows as
+ * spira_hip_conv_os, conv_ws_fused and ws_gather / gemm / scatter.) */
+int spira_hip_conv_map(int64_t num_sources, int64_t num_targets, int num_offsets, const int32_t *out_in_map,
+                       const void *sources, int row_channels, int c_in, const void *weights, const void *fragments,
+                       int c_out, int dtype, void *targets, const float *scale, const float *shift,
+                       const void *residual, int relu, hipStream_t stream);
+int spira_hip_conv_masks(int64_t num_sources, int64_t num_targets, int num_offsets, const int32_t *source_masks,
+                         const int32_t *target_masks, int dense_offsets, const int32_t *dense_map,
+                         const void *sources, int row_channels, int c_in, const void *weights, const void *fragments,
+                         int c_out, int dtype, void *targets, const float *scale, const float *shift,
+                         const void *residual, int relu, void *workspace, size_t workspace_bytes, hipStream_t stream);
+int spira_hip_conv_pairs(int64_t num_sources, int64_t num_targets, const int32_t *in_idx, const int32_t *out_idx,
+                         int rows, const int32_t *naddrs, int64_t num_pairs, int mirror_rows, int dense_offsets,
+                         const int32_t *dense_map, const void *sources, int row_channels, int c_in,
+                         const void *weights, const void *fragments, int c_out, int dtype, void *targets,
+                         const float *scale, const float *shift, const void *residual, int relu, void *workspace,
+                         size_t workspace_bytes, hipStream_t stream);
+/* Workspace bytes of conv_masks (num_pairs 0) and conv_pairs: num_offsets
+ * without the dense ones, mirrored rows included. */
+int spira_hip_conv_compact_workspace(int64_t num_sources, int64_t num_targets, int num_offsets, int64_t num_pairs,
+                                     size_t *bytes);
+
 /* Gather: buffer[padded_offsets[k] + source_masks[k, s]] = sources[s] for
  * mask entries >= 0.  padded_offsets is a HOST array of num_offsets entries.
  * (reference: Gather / PaddedGatherWarpOptimized,

@@ -48,18 +48,12 @@ struct PreparedEntry {
   hipStream_t stream = nullptr;  // the stream that allocated and wrote `prepared`
 };
 
-static std::unordered_map<const c10::TensorImpl *, PreparedEntry> &prepared_cache() {
-  static std::unordered_map<const c10::TensorImpl *, PreparedEntry> cache;
-  return cache;
-}
+using PreparedCache = std::unordered_map<const c10::TensorImpl *, PreparedEntry>;
+using PrepareFn = int (*)(const void *, int, int, int, int, void *, hipStream_t);
 
-// Returns the prepared copy of W (or an undefined tensor when the dtype needs none).
-static torch::Tensor prepared_weights(const torch::Tensor &W) {
+// The copy of W that `prepare` writes, from `cache` or made now.
+static torch::Tensor cached_copy(PreparedCache &cache, const torch::Tensor &W, size_t bytes, PrepareFn prepare) {
   const int dtype = dtype_of(W);
-  size_t bytes = 0;
-  check_rc(spira_hip_prepared_weights_bytes(W.size(0), W.size(1), W.size(2), dtype, &bytes), "prepare_weights");
-  if (bytes == 0) return torch::Tensor();
-  auto &cache = prepared_cache();
   const c10::TensorImpl *key = W.unsafeGetTensorImpl();
   auto it = cache.find(key);
   if (it != cache.end()) {
@@ -78,12 +72,48 @@ static torch::Tensor prepared_weights(const torch::Tensor &W) {
   e.version = W._version();
   e.prepared = workspace(bytes, W.device());
   e.stream = current_stream();
-  check_rc(spira_hip_prepare_weights(W.data_ptr(), W.size(0), W.size(1), W.size(2), dtype, e.prepared.data_ptr(),
-                                     current_stream()),
+  check_rc(prepare(W.data_ptr(), W.size(0), W.size(1), W.size(2), dtype, e.prepared.data_ptr(), current_stream()),
            "prepare_weights");
   auto out = e.prepared;
   cache.emplace(key, std::move(e));
   return out;
+}
+
+// Returns the prepared copy of W (or an undefined tensor when the dtype needs none).
+static torch::Tensor prepared_weights(const torch::Tensor &W) {
+  static PreparedCache cache;
+  size_t bytes = 0;
+  check_rc(spira_hip_prepared_weights_bytes(W.size(0), W.size(1), W.size(2), dtype_of(W), &bytes), "prepare_weights");
+  if (bytes == 0) return torch::Tensor();
+  return cached_copy(cache, W, bytes, &spira_hip_prepare_weights);
+}
+
+// Returns the fragment-major copy of W (the compacted kernels' weights).
+static torch::Tensor weight_fragments(const torch::Tensor &W) {
+  static PreparedCache cache;
+  size_t bytes = 0;
+  check_rc(spira_hip_fragments_bytes(W.size(0), W.size(1), W.size(2), dtype_of(W), &bytes), "prepare_fragments");
+  return cached_copy(cache, W, bytes, &spira_hip_prepare_fragments);
+}
+
+// Source rows as the compacted kernels gather them: padded with zero channels
+// to 16-byte rows, on a 16-byte boundary.
+static torch::Tensor compact_rows(const torch::Tensor &X) {
+  const int64_t v = 16 / X.element_size(), pad = (v - X.size(1) % v) % v;
+  if (pad) {
+    auto rows = torch::empty({X.size(0), X.size(1) + pad}, X.options());
+    check_rc(spira_hip_pad_rows(X.data_ptr(), X.size(0), X.size(1), X.size(1) + pad, dtype_of(X), rows.data_ptr(),
+                                current_stream()),
+             "pad_rows");
+    return rows;
+  }
+  return reinterpret_cast<uintptr_t>(X.data_ptr()) % 16 == 0 ? X : X.clone();
+}
+
+// The compacted kernels address the source rows with 31-bit byte offsets.
+static bool compact_fits(const torch::Tensor &X) {
+  const int64_t v = 16 / X.element_size();
+  return X.size(0) * ((X.size(1) + v - 1) / v * 16) < (int64_t(1) << 31);
 }
 
 // pointer to weight row `k` of W, and of its prepared copy
@@ -428,6 +458,19 @@ static OsTune tune_of(const TuneArg &t) {
   return r;
 }
 
+// An output-stationary map, or none: the identity map (targets[t] reads
+// sources[t], one offset).
+static void check_dense(const torch::Tensor *map, int64_t S, int64_t T, int K) {
+  if (map) {
+    SPIRA_CHECK_ARG(map->dim() == 2 && map->scalar_type() == torch::kInt32, "out_in_map must be 2-D int32");
+    require_device(*map, "out_in_map");
+    SPIRA_CHECK_ARG(map->size(0) >= T, "out_in_map has fewer rows than targets");
+    SPIRA_CHECK_ARG(map->size(1) == K, "out_in_map has ", map->size(1), " columns, expected ", K);
+  } else {
+    SPIRA_CHECK_ARG(S == T && K == 1, "the identity map needs as many sources as targets and one offset");
+  }
+}
+
 static bool epi_empty(const Epi &e) { return !e.scale && !e.shift && !e.residual && !e.relu; }
 
 static void run_os(const torch::Tensor *map, int64_t S, int64_t T, const torch::Tensor &X0, const torch::Tensor &W,
@@ -439,16 +482,20 @@ static void run_os(const torch::Tensor *map, int64_t S, int64_t T, const torch::
   // the split falls on a 16-channel slice (fp16), else materialised here
   const bool split = X2 && dtype == SPIRA_F16 && X0.size(1) % 32 == 0 && X2->size(1) % 8 == 0;
   const torch::Tensor X = (X2 && !split) ? torch::cat({X0, *X2}, 1) : X0;
-  const int32_t *mp = nullptr;
-  if (map) {
-    SPIRA_CHECK_ARG(map->dim() == 2 && map->scalar_type() == torch::kInt32, "out_in_map must be 2-D int32");
-    require_device(*map, "out_in_map");
-    SPIRA_CHECK_ARG(map->size(0) >= T, "out_in_map has fewer rows than targets");
-    SPIRA_CHECK_ARG(map->size(1) == K, "out_in_map has ", map->size(1), " columns, expected ", K);
-    mp = map->data_ptr<int32_t>();
-  } else {
-    // no map: the identity map (targets[t] reads sources[t], one offset)
-    SPIRA_CHECK_ARG(S == T && K == 1, "the identity map needs as many sources as targets and one offset");
+  check_dense(map, S, T, K);
+  const int32_t *mp = map ? map->data_ptr<int32_t>() : nullptr;
+  // fp32: the compacted kernel, but for small maps of rows it would have to
+  // pad first (a launch of its own: 3 -> 32 channels down-sampling 5k voxels
+  // 12 -> 16 us; 20k targets x 8 offsets and more are faster with it)
+  const bool small_unaligned = X.size(1) % 4 != 0 && T * K < 200000;
+  if (dtype == SPIRA_F32 && mp && mode == SPIRA_OUT_STORE && T > 0 && !small_unaligned && compact_fits(X)) {
+    auto F = weight_fragments(W);
+    auto Xr = compact_rows(X);
+    check_rc(spira_hip_conv_map(X.size(0), T, K, mp, Xr.data_ptr(), Xr.size(1), W.size(1), wrow_ptr(W, w0),
+                                F.data_ptr(), W.size(2), dtype, out, epi.scale, epi.shift, epi.residual, epi.relu,
+                                current_stream()),
+             "sparse_convolution_forward_os");
+    return;
   }
   // the row walk (few input channels): the map as it is and the rows unpadded
   const bool walk = tn.k.row_walk == 1 && map && dtype == SPIRA_F16 && !X2 && W.size(1) <= 16 &&
@@ -585,9 +632,7 @@ struct GsPlan {
   torch::Tensor bin, bout;
 };
 
-static GsPlan plan_gs(int64_t S, int64_t T, const torch::Tensor &source_masks, const torch::Tensor &target_masks,
-                      const torch::Tensor &nbsizes, bool half, const std::optional<double> &threshold, int cin,
-                      int cout, const torch::TensorOptions &fopt) {
+static void check_masks(int64_t S, int64_t T, const torch::Tensor &source_masks, const torch::Tensor &target_masks) {
   SPIRA_CHECK_ARG(source_masks.dim() == 2 && target_masks.dim() == 2, "masks must be 2-D");
   SPIRA_CHECK_ARG(source_masks.scalar_type() == torch::kInt32 && target_masks.scalar_type() == torch::kInt32,
                   "masks must be int32");
@@ -595,6 +640,39 @@ static GsPlan plan_gs(int64_t S, int64_t T, const torch::Tensor &source_masks, c
   require_device(target_masks, "target_masks");
   SPIRA_CHECK_ARG(source_masks.size(0) == target_masks.size(0), "source and target masks disagree on offsets");
   SPIRA_CHECK_ARG(source_masks.size(1) == S && target_masks.size(1) == T, "masks do not match S / T");
+}
+
+// Gather -> GEMM -> scatter without its buffers: the compacted kernel takes
+// each block's valid pairs from the masks (dense: a hybrid's first offsets),
+// and the per-offset sizes stay on the device.  False: features too large for
+// it (the buffered phases then run).
+static bool masks_compact(int64_t S, int64_t T, const torch::Tensor &X, const torch::Tensor &W,
+                          const torch::Tensor &source_masks, const torch::Tensor &target_masks,
+                          const torch::Tensor &nbsizes, bool half, const torch::Tensor *dense, int Kos, const Epi &e,
+                          torch::Tensor &Y) {
+  if (!compact_fits(X) || W.numel() == 0) return false;
+  check_masks(S, T, source_masks, target_masks);
+  const int Km = static_cast<int>(target_masks.size(0));
+  const int nh = half ? (Km + 1) / 2 : Km;
+  SPIRA_CHECK_ARG(nbsizes.numel() >= nh, "kernel_map_sizes has ", nbsizes.numel(), " entries, expected ", nh);
+  SPIRA_CHECK_ARG(Km <= 128, "gather: at most 128 offsets");
+  auto F = weight_fragments(W);
+  auto Xr = compact_rows(X);
+  size_t wsb = 0;
+  check_rc(spira_hip_conv_compact_workspace(S, T, Km, 0, &wsb), "gather");
+  auto ws = workspace(wsb, X.device());
+  check_rc(spira_hip_conv_masks(S, T, Km, source_masks.data_ptr<int32_t>(), target_masks.data_ptr<int32_t>(), Kos,
+                                dense ? dense->data_ptr<int32_t>() : nullptr, Xr.data_ptr(), Xr.size(1), W.size(1),
+                                W.data_ptr(), F.data_ptr(), W.size(2), dtype_of(X), Y.data_ptr(), e.scale, e.shift,
+                                e.residual, e.relu, ws.data_ptr(), wsb, current_stream()),
+           "gather");
+  return true;
+}
+
+static GsPlan plan_gs(int64_t S, int64_t T, const torch::Tensor &source_masks, const torch::Tensor &target_masks,
+                      const torch::Tensor &nbsizes, bool half, const std::optional<double> &threshold, int cin,
+                      int cout, const torch::TensorOptions &fopt) {
+  check_masks(S, T, source_masks, target_masks);
   GsPlan p;
   p.Km = static_cast<int>(target_masks.size(0));
   p.S = S;
@@ -645,12 +723,76 @@ torch::Tensor forward_ws(int64_t S, int64_t T, int64_t gather_tile, int64_t scat
                   target_masks.size(0));
   const int Km = static_cast<int>(target_masks.size(0));
   const bool half = (Km % 2 == 1) && S == T;
-  auto p = plan_gs(S, T, source_masks, target_masks, nbsizes, half, threshold, W.size(1), W.size(2), X.options());
   auto Y = torch::empty({T, W.size(2)}, X.options());
   auto s = current_stream();
+  const Epi e = epi_of(scale, shift, residual, relu, T, W.size(2), X);
+  if (masks_compact(S, T, X, W, source_masks, target_masks, nbsizes, half, nullptr, 0, e, Y)) return Y;
+  auto p = plan_gs(S, T, source_masks, target_masks, nbsizes, half, threshold, W.size(1), W.size(2), X.options());
   gs_gather(p, X, s);
   gs_gemm(p, W, 0, s);
-  gs_scatter(p, W.size(2), dtype_of(X), nullptr, Y.data_ptr(), s, epi_of(scale, shift, residual, relu, T, W.size(2), X));
+  gs_scatter(p, W.size(2), dtype_of(X), nullptr, Y.data_ptr(), s, e);
+  return Y;
+}
+
+// Whether a pair list goes to the compacted kernel or to the fused pass with
+// its atomics.  The compacted kernel reads an offset's weights once per 64
+// targets, so it wants a few pairs of each offset there: d = pairs per offset
+// and 64 targets.  fp16 (measured, us, fused -> compacted): 64 -> 64 channels
+// at d = 3.3 28.9 -> 29.9, at 5 101 -> 66, at 15 73 -> 35; 256 -> 256 at 3.3
+// 89 -> 127, at 5 352 -> 348, at 15 258 -> 157; outputs of 32 columns and
+// fewer are faster fused at every d (their atomics are few: 16 -> 16 at d = 15
+// 24 -> 34).  fp32's fused pass runs on the vector ALU: it wins only small
+// layers (100M multiply-adds at 27 offsets 40 -> 43, 245M 86 -> 59, 800M 535 ->
+// 70; with 125 offsets 120M 48 -> 76, 390M 214 -> 186).
+static bool pairs_compact_pays(int64_t pairs, int64_t T, int64_t K, int64_t cin, int64_t cout, int dtype) {
+  if (dtype == SPIRA_F32)
+    return static_cast<double>(pairs) * cin * cout >= 1e8 * std::max(1.0, static_cast<double>(K) / 32);
+  const double d = 64.0 * pairs / (static_cast<double>(std::max<int64_t>(T, 1)) * K);
+  return cout > 32 && d >= (cin > 128 ? 6.5 : 3.6);
+}
+
+static void check_pairs(const torch::Tensor &naddrs, const torch::Tensor &qnaddrs, const torch::Tensor &nbmaps,
+                        int64_t mapsize, int weight_rows, const torch::Tensor &W, int dtype) {
+  SPIRA_CHECK_ARG(nbmaps.dim() == 2 && nbmaps.size(0) == 2, "nbmaps must be [2, P]");
+  SPIRA_CHECK_ARG(nbmaps.size(1) == mapsize, "nbmaps holds ", nbmaps.size(1), " pairs, mapsize is ", mapsize);
+  require_device(nbmaps, "nbmaps");
+  require_device(naddrs, "naddrs");
+  require_device(qnaddrs, "qnaddrs");
+  SPIRA_CHECK_ARG(naddrs.size(0) > 1 || mapsize == 0, "conv_ws_fused: rows must be positive");
+  SPIRA_CHECK_ARG(weight_rows <= W.size(0), "conv_ws_fused: weight rows out of range");
+  SPIRA_CHECK_ARG(dtype != SPIRA_F16 || naddrs.size(0) - 1 <= 128 || mapsize == 0,
+                  "conv_ws_fused: at most 128 offset rows");
+}
+
+// The pair list through the compacted kernel: entry rows by target, then each
+// block's valid pairs (dense: a hybrid's first offsets).  None: the fused pass
+// runs instead (pairs_compact_pays, or features too large).
+static std::optional<torch::Tensor> pairs_compact(int64_t S, int64_t T, const torch::Tensor &X, const torch::Tensor &W,
+                          const torch::Tensor &naddrs, const torch::Tensor &qnaddrs, const torch::Tensor &nbmaps,
+                          int64_t mapsize, bool transpose, int mirror_rows, const torch::Tensor *dense, int Kos,
+                          const Epi &e) {
+  const int rows = static_cast<int>(naddrs.size(0) - 1);
+  if (!compact_fits(X) || W.numel() == 0 || mapsize >= (int64_t(1) << 29)) return std::nullopt;
+  // (about T pairs in a self-mirrored centre row, taken once, and in a
+  // hybrid's dense offsets)
+  const int64_t pairs = (mirror_rows > 0 ? 2 : 1) * mapsize - (mirror_rows % 2 == 1 ? T : 0) + (Kos > 0 ? T : 0);
+  if (!pairs_compact_pays(pairs, T, Kos + std::max(mirror_rows, rows), W.size(1), W.size(2), dtype_of(X)))
+    return std::nullopt;
+  check_pairs(naddrs, qnaddrs, nbmaps, mapsize, Kos + std::max(mirror_rows, rows), W, dtype_of(X));
+  const int32_t *base = nbmaps.data_ptr<int32_t>();
+  const int32_t *imap = transpose ? base + mapsize : base;
+  const int32_t *omap = transpose ? base : base + mapsize;
+  auto Y = torch::empty({T, W.size(2)}, X.options());
+  auto F = weight_fragments(W);
+  auto Xr = compact_rows(X);
+  size_t wsb = 0;
+  check_rc(spira_hip_conv_compact_workspace(S, T, std::max(mirror_rows, rows), mapsize, &wsb), "ws_merged");
+  auto ws = workspace(wsb, X.device());
+  check_rc(spira_hip_conv_pairs(S, T, imap, omap, rows, naddrs.data_ptr<int32_t>(), mapsize, mirror_rows, Kos,
+                                dense ? dense->data_ptr<int32_t>() : nullptr, Xr.data_ptr(), Xr.size(1), W.size(1),
+                                W.data_ptr(), F.data_ptr(), W.size(2), dtype_of(X), Y.data_ptr(), e.scale, e.shift,
+                                e.residual, e.relu, ws.data_ptr(), wsb, current_stream()),
+           "sparse_convolution_forward_ws_merged");
   return Y;
 }
 
@@ -659,12 +801,8 @@ static void ws_fused_into(int64_t S, int64_t T, const torch::Tensor &X, const to
                           const torch::Tensor &naddrs, const torch::Tensor &qnaddrs, const torch::Tensor &nbmaps,
                           int64_t mapsize, int64_t qmapsize, bool transpose, int woff, int mirror_rows,
                           float *acc) {
-  SPIRA_CHECK_ARG(nbmaps.dim() == 2 && nbmaps.size(0) == 2, "nbmaps must be [2, P]");
-  SPIRA_CHECK_ARG(nbmaps.size(1) == mapsize, "nbmaps holds ", nbmaps.size(1), " pairs, mapsize is ", mapsize);
-  require_device(nbmaps, "nbmaps");
-  require_device(naddrs, "naddrs");
-  require_device(qnaddrs, "qnaddrs");
   const int rows = static_cast<int>(naddrs.size(0) - 1);
+  check_pairs(naddrs, qnaddrs, nbmaps, mapsize, woff + std::max(mirror_rows, rows), W, dtype_of(X));
   const int32_t *base = nbmaps.data_ptr<int32_t>();
   const int32_t *imap = transpose ? base + mapsize : base;
   const int32_t *omap = transpose ? base : base + mapsize;
@@ -697,9 +835,11 @@ torch::Tensor forward_ws_merged(int64_t S, int64_t T, const torch::Tensor &X, co
   // mirrored pass for submanifold maps with an odd kernel volume
   // (sparse_convolution.cu:1287-1293)
   const int mirror = (S == T && K % 2 == 1) ? K : 0;
+  const Epi e = epi_of(scale, shift, residual, relu, T, W.size(2), X);
+  if (auto y = pairs_compact(S, T, X, W, naddrs, qnaddrs, nbmaps, mapsize, transpose, mirror, nullptr, 0, e)) return *y;
   auto acc = torch::zeros({T, W.size(2)}, X.options().dtype(torch::kFloat));
   ws_fused_into(S, T, X, W, naddrs, qnaddrs, nbmaps, mapsize, qmapsize, transpose, 0, mirror, acc.data_ptr<float>());
-  return finish_acc(acc, X, epi_of(scale, shift, residual, relu, T, W.size(2), X));
+  return finish_acc(acc, X, e);
 }
 
 // (reference: CUDASparseConvolutionForward_HS, :254-342)
@@ -716,16 +856,18 @@ torch::Tensor forward_hs(int64_t S, int64_t T, int64_t gather_tile, int64_t scat
   const int Kws = static_cast<int>(target_masks.size(0));
   const int Kos = out_in_map.has_value() ? static_cast<int>(out_in_map->size(1)) : 1;
   SPIRA_CHECK_ARG(W.size(0) == Kws + Kos, "weights have ", W.size(0), " offsets, expected ", Kws + Kos);
-  auto acc = torch::empty({T, W.size(2)}, X.options().dtype(torch::kFloat));
-  run_os(out_in_map.has_value() ? &*out_in_map : nullptr, S, T, X, W, 0, Kos, acc.data_ptr<float>(),
-         SPIRA_OUT_STORE_F32);
-  auto p = plan_gs(S, T, source_masks, target_masks, nbsizes, true, threshold, W.size(1), W.size(2), X.options());
+  const torch::Tensor *dense = out_in_map.has_value() ? &*out_in_map : nullptr;
   auto Y = torch::empty({T, W.size(2)}, X.options());
   auto s = current_stream();
+  const Epi e = epi_of(scale, shift, residual, relu, T, W.size(2), X);
+  check_dense(dense, S, T, Kos);
+  if (masks_compact(S, T, X, W, source_masks, target_masks, nbsizes, true, dense, Kos, e, Y)) return Y;
+  auto acc = torch::empty({T, W.size(2)}, X.options().dtype(torch::kFloat));
+  run_os(dense, S, T, X, W, 0, Kos, acc.data_ptr<float>(), SPIRA_OUT_STORE_F32);
+  auto p = plan_gs(S, T, source_masks, target_masks, nbsizes, true, threshold, W.size(1), W.size(2), X.options());
   gs_gather(p, X, s);
   gs_gemm(p, W, Kos, s);
-  gs_scatter(p, W.size(2), dtype_of(X), acc.data_ptr<float>(), Y.data_ptr(), s,
-             epi_of(scale, shift, residual, relu, T, W.size(2), X));
+  gs_scatter(p, W.size(2), dtype_of(X), acc.data_ptr<float>(), Y.data_ptr(), s, e);
   return Y;
 }
 
@@ -740,11 +882,14 @@ torch::Tensor forward_hs_merged(int64_t S, int64_t T, const torch::Tensor &X, co
   const int Kws = static_cast<int>((naddrs.size(0) - 1) * 2);
   const int Kos = out_in_map.has_value() ? static_cast<int>(out_in_map->size(1)) : 1;
   SPIRA_CHECK_ARG(W.size(0) == Kws + Kos, "weights have ", W.size(0), " offsets, expected ", Kws + Kos);
+  const torch::Tensor *dense = out_in_map.has_value() ? &*out_in_map : nullptr;
+  const Epi e = epi_of(scale, shift, residual, relu, T, W.size(2), X);
+  check_dense(dense, S, T, Kos);
+  if (auto y = pairs_compact(S, T, X, W, naddrs, qnaddrs, nbmaps, mapsize, transpose, Kws, dense, Kos, e)) return *y;
   auto acc = torch::empty({T, W.size(2)}, X.options().dtype(torch::kFloat));
-  run_os(out_in_map.has_value() ? &*out_in_map : nullptr, S, T, X, W, 0, Kos, acc.data_ptr<float>(),
-         SPIRA_OUT_STORE_F32);
+  run_os(dense, S, T, X, W, 0, Kos, acc.data_ptr<float>(), SPIRA_OUT_STORE_F32);
   ws_fused_into(S, T, X, W, naddrs, qnaddrs, nbmaps, mapsize, qmapsize, transpose, Kos, Kws, acc.data_ptr<float>());
-  return finish_acc(acc, X, epi_of(scale, shift, residual, relu, T, W.size(2), X));
+  return finish_acc(acc, X, e);
 }
 
 // ---- selector probes: time one phase of the gather-GEMM-scatter path ----

@@ -1,0 +1,135 @@
+"""The compacted convolution kernels (masks, pair lists, fp32 maps) at the
+edges of their tiles: targets around a block of 64, offsets around a chunk of
+32, channels around the 16-byte row and the column tiles, empty and full maps,
+pairs in any order and repeated pairs.  Against a float64 sum over the pairs.
+
+Tolerance, max |error| / RMS(reference): fp16 stores round to 2^-11 of a value
+that may be 6 x RMS (3e-3) -> 4e-3; fp32 sums of up to 8000 products, error
+growth ~ sqrt(n) 2^-24 of the terms' norm -> 1e-5 (the fp32 bar)."""
+import numpy as np
+import pytest
+import torch
+
+from spira_amd.nn import functional as F
+
+from helpers import np_, rel_err
+
+pytestmark = pytest.mark.gpu
+
+TOL = {torch.float16: 4e-3, torch.float32: 1e-5}
+#        S    T    K  cin cout  density
+SHAPES = [(1, 1, 1, 3, 1, 1.0), (70, 63, 8, 4, 16, 0.5), (70, 64, 27, 16, 17, 0.3), (90, 65, 33, 20, 48, 0.4),
+          (130, 129, 31, 33, 64, 0.0), (200, 128, 32, 64, 65, 1.0), (300, 200, 65, 96, 97, 0.2),
+          (64, 190, 125, 24, 40, 0.3), (150, 100, 27, 160, 130, 0.5), (150, 100, 27, 256, 48, 0.6)]
+
+
+def _lists(S, T, K, density, seed):
+    """Per offset: distinct sources and distinct targets, paired at random."""
+    rng = np.random.default_rng(seed)
+    out = []
+    for _ in range(K):
+        n = int(round(density * min(S, T)))
+        out.append((rng.permutation(S)[:n].astype(np.int32), rng.permutation(T)[:n].astype(np.int32)))
+    return out
+
+
+def _data(S, T, K, cin, cout, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    X = torch.randn(S, cin, generator=g).to(dtype)
+    W = (torch.randn(K, cin, cout, generator=g) / np.sqrt(cin)).to(dtype)
+    epi = (torch.rand(cout, generator=g) + 0.5, torch.randn(cout, generator=g),
+           torch.randn(T, cout, generator=g).to(dtype), True)
+    return X, W, epi
+
+
+def _ref(lists, T, X, W, epi=None):
+    X, W = X.double().numpy(), W.double().numpy()
+    y = np.zeros((T, W.shape[2]))
+    for k, (s, t) in enumerate(lists):
+        np.add.at(y, t, X[s] @ W[k])
+    if epi is not None:
+        scale, shift, res, _ = epi
+        y = np.maximum(y * scale.double().numpy() + shift.double().numpy() + res.double().numpy(), 0)
+    return y
+
+
+def _dev(epi, dev):
+    return tuple(v.to(dev) if isinstance(v, torch.Tensor) else v for v in epi)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("S,T,K,cin,cout,density", SHAPES)
+def test_masks(dev, dtype, S, T, K, cin, cout, density):
+    lists = _lists(S, T, K, density, S + K)
+    X, W, epi = _data(S, T, K, cin, cout, dtype, K)
+    sm, tm = np.full((K, S), -1, np.int32), np.full((K, T), -1, np.int32)
+    for k, (s, t) in enumerate(lists):
+        sm[k, s] = tm[k, t] = np.arange(len(s))
+    sizes = torch.tensor([len(s) for s, _ in lists], dtype=torch.int32, device=dev)
+    args = (S, T, X.to(dev), W.to(dev), torch.from_numpy(sm).to(dev), torch.from_numpy(tm).to(dev), sizes, 16, 16)
+    y = F.sparse_convolution_forward_ws(*args)
+    assert rel_err(np_(y.float()), _ref(lists, T, X, W)) <= TOL[dtype]
+    y2 = F.sparse_convolution_forward_ws(*args, epilogue=_dev(epi, dev))
+    assert rel_err(np_(y2.float()), _ref(lists, T, X, W, epi)) <= TOL[dtype]
+    assert torch.equal(y, F.sparse_convolution_forward_ws(*args))  # (sums in a fixed order)
+
+
+@pytest.mark.parametrize("S,T,K,cin,cout,density", SHAPES)
+def test_fp32_map(dev, S, T, K, cin, cout, density):
+    lists = _lists(S, T, K, density, S + K)
+    X, W, epi = _data(S, T, K, cin, cout, torch.float32, K)
+    m = np.full(((T + 127) // 128 * 128, K), -1, np.int32)
+    for k, (s, t) in enumerate(lists):
+        m[t, k] = s
+    y = F.sparse_convolution_forward_os(S, T, torch.from_numpy(m).to(dev), X.to(dev), W.to(dev),
+                                        epilogue=_dev(epi, dev))
+    assert rel_err(np_(y), _ref(lists, T, X, W, epi)) <= TOL[torch.float32]
+
+
+@pytest.mark.parametrize("repeat", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("S,T,K,cin,cout", [(2100, 2000, 27, 64, 64), (1500, 1400, 8, 96, 100), (900, 901, 40, 128, 48)])
+def test_pairs(dev, dtype, S, T, K, cin, cout, repeat):
+    """Dense enough for the compacted kernel; rows of pairs shuffled, and with
+    `repeat` every 50th pair given twice (both count)."""
+    lists = _lists(S, T, K, 0.6, S + K)
+    if repeat:
+        lists = [(np.concatenate([s, s[::50]]), np.concatenate([t, t[::50]])) for s, t in lists]
+    X, W, epi = _data(S, T, K, cin, cout, dtype, K)
+    sizes = np.array([len(s) for s, _ in lists])
+    naddrs = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    qn = np.concatenate([[0], np.cumsum((sizes + 127) // 128 * 128)]).astype(np.int32)
+    nb = np.stack([np.concatenate([s for s, _ in lists]), np.concatenate([t for _, t in lists])]).astype(np.int32)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    y = F.sparse_convolution_forward_ws_merged(S, T, X.to(dev), W.to(dev), d(naddrs), d(qn), d(nb), nb.shape[1],
+                                               int(qn[-1]), epilogue=_dev(epi, dev))
+    assert rel_err(np_(y.float()), _ref(lists, T, X, W, epi)) <= TOL[dtype]
+    # transposed: sources and targets exchanged
+    back = [(t, s) for s, t in lists]
+    X2, _, _ = _data(T, S, K, cin, cout, dtype, K + 1)
+    y = F.sparse_convolution_forward_ws_merged(T, S, X2.to(dev), W.to(dev), d(naddrs), d(qn), d(nb), nb.shape[1],
+                                               int(qn[-1]), True)
+    assert rel_err(np_(y.float()), _ref(back, S, X2, W)) <= TOL[dtype]
+
+
+def test_values_stay_in_their_rows(dev):
+    """An infinity and a NaN reach exactly the targets that have them as a
+    neighbour, and unaligned views of the features are taken as they are."""
+    S = T = 150
+    lists = _lists(S, T, 27, 0.2, 5)
+    X, W, _ = _data(S, T, 27, 40, 36, torch.float32, 3)
+    m = np.full((256, 27), -1, np.int32)
+    for k, (s, t) in enumerate(lists):
+        m[t, k] = s
+    md = torch.from_numpy(m).to(dev)
+    flat = torch.empty(S * 40 + 1, device=dev)
+    view = flat[1:].view(S, 40)
+    view.copy_(X)
+    assert rel_err(np_(F.sparse_convolution_forward_os(S, T, md, view, W.to(dev))), _ref(lists, T, X, W)) <= 1e-5
+    X[7], X[90] = float("inf"), float("nan")
+    y = np_(F.sparse_convolution_forward_os(S, T, md, X.to(dev), W.to(dev)))
+    touched = np.zeros(T, bool)
+    for s, t in lists:
+        touched[t[(s == 7) | (s == 90)]] = True
+    assert not np.isfinite(y[touched]).any(axis=1).any() or np.isnan(y[touched]).any(axis=1).all()
+    assert np.isfinite(y[~touched]).all()
