@@ -1868,14 +1868,25 @@ static inline int bm_for(int wn) {
 // offsets per split: small layers split their offsets so that the grid
 // covers the chip; a split never exceeds 128 offsets (the block's 128-bit
 // active-offset set).  splits > 0: that many splits, as asked.
-static int choose_jper(int64_t blocks_xy, int Kc, int cus, int splits = 0) {
+//   Up to 27 offsets: only where two or more CUs are there per block; one
+// split more than fills the chip costs its atomics and finalize pass (32 ->
+// 32, 20k voxels, 157 blocks: 16.2 us with two splits, 13.2 with one; 64 ->
+// 64, 14k voxels 18.9 -> 15.5).
+//   More offsets: a block runs over a hundred dependent steps, so they split
+// until two blocks share a CU (2.5 of 32 columns), at most into eighths, and
+// inputs of 96 channels and more into thirds up to 1.25 blocks per CU.  125
+// offsets, 20k voxels, 157 row tiles: 64 -> 64 57 -> 41 us, 96 -> 96 101 ->
+// 69, 128 -> 128 120 -> 93, 16 -> 16 30 -> 22; 128 -> 128 at 263 row tiles
+// 190 -> 160.
+static int choose_jper(int64_t blocks_xy, int Kc, int CinP, int wn, int cus, int splits = 0) {
   int jper = Kc;
-  if (splits > 0) {
-    jper = static_cast<int>(div_up(Kc, std::min(splits, Kc)));
-  } else if (blocks_xy < cus && Kc > 1) {
-    const int64_t n = std::min<int64_t>(Kc, div_up(cus, blocks_xy));
-    jper = static_cast<int>(div_up(Kc, n));
-  }
+  int64_t n = 1;
+  if (splits > 0) n = std::min(splits, Kc);
+  else if (Kc > ring::kMapTileK && blocks_xy < cus)
+    n = std::min<int64_t>((wn == 1 ? 5 : 4) * cus / (2 * blocks_xy), std::max<int64_t>(8, cus / blocks_xy));
+  else if (Kc > ring::kMapTileK && CinP >= 96 && 4 * blocks_xy <= 5 * static_cast<int64_t>(cus)) n = 3;
+  else if (Kc > 1 && blocks_xy < cus) n = cus / blocks_xy;
+  if (n > 1) jper = static_cast<int>(div_up(Kc, std::min<int64_t>(n, Kc)));
   return std::min(jper, 128);
 }
 
@@ -1982,21 +1993,40 @@ static int os_nks(int CinP, int wn, int64_t blocks, int cus, int step_channels) 
 }
 
 // Column-tile width of the output-stationary kernel: the widest tile, made
-// narrower once (more column blocks, each re-gathering its rows) when the
-// grid has fewer than SPIRA_OS_MIN_BLOCKS (default 1) blocks per CU; a grid
-// still short of the CUs then splits its offsets (choose_jper).  (Measured
-// on the config-4 layers: s8 128 -> 128, 134 row blocks, is fastest with
-// one halving (42.9 us, 46.7 us without); s16 256 -> 256, 32 row blocks,
-// took 53.0 us narrowed down to 32-column tiles against 34.8 us without,
-// as every narrowing multiplies the gathered rows.  More than one block per
-// CU this way, or by more offset splits, costs more in re-gathered rows /
-// atomics than the added occupancy returns.)
-static int os_wn(int64_t num_targets, int c_out, int cus, int col_tile) {
+// narrower (more column blocks, each re-gathering its rows) when the grid is
+// short of the chip; a grid still short of the CUs then splits its offsets
+// (choose_jper).  Where the lines lie:
+//   Up to 8 offsets: one block per CU.
+//   9 to 27 offsets: 96 columns at 40 % of the CUs (31k voxels, 243 blocks:
+// 25.9 us wide, 37.3 narrow; 110 blocks 23.9 / 24.8), 64 columns and wide
+// inputs at half of them (128 -> 128, 243 blocks 32.4 / 37.2; 110 blocks 29.2
+// / 23.1), else at one block per CU (64 -> 128, 204 blocks 23.7 / 21.9).  A
+// second step down to 32 columns only where it fills the chip without a split
+// (128 -> 128, 7k voxels, 220 blocks: 22.3 -> 18.6 us); further, every
+// narrowing multiplies the gathered rows (256 -> 256, 32 row blocks: 53.0 us
+// at 32 columns, 34.8 at 64 and two splits).
+//   More offsets: split rather than narrow (125 offsets, 96 -> 96, 157 blocks
+// 101 -> 69 us), but for 128 columns of at most 64 channels, whose narrow
+// tiles pack two offsets per step (243 blocks 85 / 74), and of more channels
+// below a quarter of the CUs (55 blocks 48.6 / 43.4).
+//   Index-order layers of 256 columns and more whose 128-column blocks are
+// just over one per CU take 96-column tiles, which fill the last round (20k
+// voxels, 314 blocks: 89 -> 70 us).
+static int os_wn(int64_t num_targets, int c_out, int cus, int col_tile, int Kc, int CinP, bool ordered) {
   if (col_tile == 32 || col_tile == 64 || col_tile == 96 || col_tile == 128) return col_tile / 32;
-  int wn = wn_for(c_out);
-  const int64_t bx = div_up(num_targets, bm_for(1));
-  if (wn > 1 && bx * div_up(pad_out(c_out), 32 * wn) < cus) wn = wn == 3 ? 1 : wn / 2;
-  return wn;
+  const int wn = wn_for(c_out);
+  const int64_t rows = div_up(num_targets, bm_for(1)), cols = pad_out(c_out);
+  const int64_t blocks = rows * div_up(cols, 32 * wn);
+  const bool many = Kc > ring::kMapTileK, mid = Kc > 8 && !many;
+  int64_t least = cus;
+  if (many) least = wn < 4 ? 0 : CinP <= 64 ? cus : cus / 4;
+  else if (Kc > 8 && !ordered && c_out >= 256 && blocks > cus && 4 * blocks <= 5 * static_cast<int64_t>(cus)) return 3;
+  else if (mid && wn == 3) least = cus * 2 / 5;
+  else if (mid && (wn == 2 || CinP >= 96)) least = cus / 2;
+  if (wn == 1 || blocks >= least) return wn;
+  if (wn == 3) return 1;
+  const int64_t half = rows * div_up(cols, 16 * wn);
+  return wn == 4 && mid && 2 * half < cus && 10 * half >= 3 * static_cast<int64_t>(cus) ? 1 : wn / 2;
 }
 
 // A third ring stage (two steps of gathers in flight instead of one) for
@@ -2062,15 +2092,15 @@ struct OsPlan {
 };
 
 static OsPlan plan_os(int64_t T, int Kc, int Cin, int CinP, bool cat, int Cout, bool has_map, bool native_store,
-                      const spira_hip_os_tuning_t &tn) {
+                      const spira_hip_os_tuning_t &tn, bool ordered = false) {
   OsPlan pl{};
   const int cus = device_cu_count();
-  pl.wn = os_wn(T, Cout, cus, tn.col_tile);
+  pl.wn = os_wn(T, Cout, cus, tn.col_tile, Kc, CinP, ordered);
   pl.bm = bm_for(pl.wn);
   pl.gx = div_up(T, pl.bm);
   pl.gy = div_up(pad_out(Cout), 32 * pl.wn);
-  // small layers (fewer blocks than CUs) split their offsets over grid z
-  pl.jper = choose_jper(pl.gx * pl.gy, Kc, cus, tn.offset_splits);
+  // small layers split their offsets over grid z
+  pl.jper = choose_jper(pl.gx * pl.gy, Kc, CinP, pl.wn, cus, tn.offset_splits);
   pl.splits = static_cast<int>(div_up(Kc, pl.jper));
   pl.aligned = Cin % 8 == 0;
   pl.xcd = tn.block_order;
@@ -2266,13 +2296,15 @@ int spira_hip_prepare_weights(const void *weights, int num_offsets, int c_in, in
 
 int spira_hip_conv_os_workspace(int64_t num_targets, int num_offsets, int c_in, int c_out, int dtype, int out_mode,
                                 const spira_hip_os_tuning_t *tuning, size_t *bytes) {
-  (void)c_in;
   *bytes = 0;
   const spira_hip_os_tuning_t tn = tuning_of(tuning);
   if (int rc = check_tuning(tn)) return rc;
   if (!mfma_path(dtype) || out_mode != SPIRA_OUT_STORE || num_targets <= 0) return kOk;
   const OsPlan pl = plan_os(num_targets, num_offsets, c_in, pad_in(c_in), false, c_out, true, true, tn);
-  if (pl.splits > 1)
+  // (a concatenation's plan goes by the channels of both parts, of which c_in
+  // may name the first alone: splits of the widest input count too)
+  const OsPlan wide = plan_os(num_targets, num_offsets, 512, 512, false, c_out, true, true, tn);
+  if (pl.splits > 1 || wide.splits > 1)
     *bytes = static_cast<size_t>(num_targets) * c_out * sizeof(float);
   *bytes = std::max(*bytes, pl.bal_bytes());
   return kOk;
@@ -2348,7 +2380,7 @@ static int conv_os_impl(int64_t num_targets, int num_offsets, const int32_t *out
     SPIRA_HIP_REQUIRE(prepared != nullptr, "conv_os: fp16 needs prepared weights (spira_hip_prepare_weights)");
     const int cin_all = c_in + c_in2;
     OsPlan pl = plan_os(num_targets, num_offsets, cin_all, pad_in(cin_all), c_in2 > 0, c_out,
-                        out_in_map != nullptr, out_mode == SPIRA_OUT_STORE, tn);
+                        out_in_map != nullptr, out_mode == SPIRA_OUT_STORE, tn, group_masks != nullptr);
     // (the one-wave-per-SIMD build only for row-ordered maps: their longest
     // tiles come first, so blocks past the first round are short ones)
     if (pl.da == 2 && !group_masks) pl.da = 1;

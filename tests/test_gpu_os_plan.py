@@ -1,0 +1,54 @@
+"""Column tiles and offset splits of the output-stationary kernel on both
+sides of the lines where they change (256 CUs): the plan, and the layer's
+output against a float64 sum over the map.
+
+Tolerance, max |error| / RMS(reference): the fp16 store rounds to 2^-11 of a
+value that may be 6 x RMS (3e-3), and the fp32 sums of the splits add far less
+-> 4e-3."""
+import numpy as np
+import pytest
+import torch
+
+from spira_amd.nn import functional as F
+from spira_amd.nn.functional import _native
+
+from helpers import np_, rel_err
+
+#         T    K  cin cout  (column tile, splits)
+PLANS = [(400, 8, 32, 128, 64, 8), (16300, 27, 32, 32, 32, 2), (16500, 27, 32, 32, 32, 1),
+         (12900, 27, 128, 128, 64, 1), (16500, 27, 128, 128, 128, 1), (7000, 27, 128, 128, 32, 1),
+         (12900, 27, 64, 96, 32, 1), (13000, 27, 64, 96, 96, 2), (20000, 27, 64, 256, 96, 1),
+         (20600, 27, 64, 256, 128, 1), (700, 125, 16, 16, 32, 42), (16300, 125, 16, 16, 32, 5),
+         (32600, 125, 32, 64, 64, 2), (32900, 125, 32, 64, 64, 1), (8000, 125, 96, 128, 64, 4),
+         (8300, 125, 96, 128, 128, 7), (40900, 125, 96, 64, 64, 3), (41100, 125, 96, 64, 64, 1)]
+
+
+@pytest.mark.parametrize("T,K,cin,cout,tile,splits", PLANS)
+def test_plan(T, K, cin, cout, tile, splits):
+    if torch.cuda.is_available() and torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the lines are stated for 256 CUs")
+    plan = _native._C.conv_os_plan(T, K, cin, 0, cout, True)
+    assert (plan[0], plan[2]) == (tile, splits)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,K,cin,cout,tile,splits", PLANS)
+def test_output(dev, T, K, cin, cout, tile, splits):
+    g = torch.Generator().manual_seed(T)
+    S = T // 2 + 1
+    m = torch.randint(-2 * S, S, (T, K), generator=g, dtype=torch.int32).clamp_(min=-1)
+    m[T - 130:T - 1] = -1  # an empty row group and more
+    X = torch.randn(S, cin, generator=g).half().to(dev)
+    W = (torch.randn(K, cin, cout, generator=g) / np.sqrt(9 * cin)).half().to(dev)
+    m = torch.nn.functional.pad(m, (0, 0, 0, -T % 128), value=-1).to(dev)
+    y = F.sparse_convolution_forward_os(S, T, m, X, W)
+    rows = torch.cat([torch.arange(0, min(T, 400)), torch.arange(max(0, T - 400), T)]).unique().to(dev)
+    Xz = torch.cat([X.double(), torch.zeros(1, cin, device=dev, dtype=torch.float64)])
+    ref = torch.zeros(len(rows), cout, device=dev, dtype=torch.float64)
+    for k in range(K):
+        ref += Xz[m[rows, k].long()] @ W[k].double()
+    assert rel_err(np_(y[rows].float()), np_(ref)) <= 4e-3
+    # a concatenated input plans by the channels of both parts
+    if cin > 32 and cin % 32 == 0:
+        y2 = F.sparse_convolution_forward_os(S, T, m, X[:, :32].contiguous(), W, sources2=X[:, 32:].contiguous())
+        assert rel_err(np_(y2[rows].float()), np_(ref)) <= 4e-3
