@@ -572,8 +572,10 @@ static void launch_n(hipStream_t s, const Entries &en, int64_t T, int K, const L
   } else if constexpr (sizeof(FT) == 4) {
     SPIRA_PAIR_CALL(4, 32, 2, occ4);
   } else {
+    // (96 columns of 96 channels and more: eight waves, two of them idle; 128
+    // -> 96 on 90k LiDAR voxels 123 us with six, 95 with eight)
     if (l.Cout <= 64) SPIRA_PAIR_CALL(4, 32, 2, occ4);
-    else if (l.Cout <= 96) SPIRA_PAIR_CALL(6, 32, 3, 3);
+    else if (l.Cout <= 96 && PITCH < 256) SPIRA_PAIR_CALL(6, 32, 3, 3);
     else SPIRA_PAIR_CALL(8, 32, 3, 4);
   }
 #undef SPIRA_PAIR_CALL

@@ -1868,24 +1868,35 @@ static inline int bm_for(int wn) {
 // offsets per split: small layers split their offsets so that the grid
 // covers the chip; a split never exceeds 128 offsets (the block's 128-bit
 // active-offset set).  splits > 0: that many splits, as asked.
-//   Up to 27 offsets: only where two or more CUs are there per block; one
-// split more than fills the chip costs its atomics and finalize pass (32 ->
-// 32, 20k voxels, 157 blocks: 16.2 us with two splits, 13.2 with one; 64 ->
-// 64, 14k voxels 18.9 -> 15.5).
+//   Up to 27 offsets: where two or more CUs are there per block (96-column
+// blocks: more); one split more than fills the chip costs its atomics and
+// finalize pass (32 -> 32, 20k voxels, 157 blocks: 16.2 us with two splits,
+// 13.2 with one; 32 -> 96, 122 blocks 25.1 / 17.8).  Long blocks (256
+// channels and more, or a last 16 of them in steps of their own) until
+// nearly every CU has one (48 -> 16, 250 blocks: 18.8 us with two, 20.9 with
+// one).
 //   More offsets: a block runs over a hundred dependent steps, so they split
 // until two blocks share a CU (2.5 of 32 columns), at most into eighths, and
 // inputs of 96 channels and more into thirds up to 1.25 blocks per CU.  125
 // offsets, 20k voxels, 157 row tiles: 64 -> 64 57 -> 41 us, 96 -> 96 101 ->
 // 69, 128 -> 128 120 -> 93, 16 -> 16 30 -> 22; 128 -> 128 at 263 row tiles
-// 190 -> 160.
+// 190 -> 160.  Not wide tiles of up to 32 channels on 70 % of the CUs, which
+// pack four offsets per step unsplit (16 -> 64, 250 blocks 48.0 / 42.2).
 static int choose_jper(int64_t blocks_xy, int Kc, int CinP, int wn, int cus, int splits = 0) {
   int jper = Kc;
   int64_t n = 1;
-  if (splits > 0) n = std::min(splits, Kc);
-  else if (Kc > ring::kMapTileK && blocks_xy < cus)
-    n = std::min<int64_t>((wn == 1 ? 5 : 4) * cus / (2 * blocks_xy), std::max<int64_t>(8, cus / blocks_xy));
-  else if (Kc > ring::kMapTileK && CinP >= 96 && 4 * blocks_xy <= 5 * static_cast<int64_t>(cus)) n = 3;
-  else if (Kc > 1 && blocks_xy < cus) n = cus / blocks_xy;
+  if (splits > 0) {
+    n = std::min(splits, Kc);
+  } else if (Kc > ring::kMapTileK) {
+    const int64_t most = std::max<int64_t>(CinP >= 64 && wn == 2 ? 6 : 8, cus / blocks_xy);
+    if (CinP <= 32 && wn >= 2 && blocks_xy * 10 > static_cast<int64_t>(cus) * 7) n = 1;
+    else if (blocks_xy < cus) n = std::min<int64_t>((wn == 1 && CinP <= 32 ? 5 : 4) * cus / (2 * blocks_xy), most);
+    else if (CinP >= 96 && 4 * blocks_xy <= 5 * static_cast<int64_t>(cus)) n = 3;
+  } else if (Kc > 1 && blocks_xy < cus) {
+    const bool deep = CinP >= 256 || (CinP > 16 && CinP % 32 != 0);
+    const int64_t limit = deep ? (wn == 1 ? cus : cus * 3 / 5) : wn == 3 ? cus * 2 / 5 : cus / 2;
+    if (blocks_xy <= limit) n = div_up(cus, blocks_xy);
+  }
   if (n > 1) jper = static_cast<int>(div_up(Kc, std::min<int64_t>(n, Kc)));
   return std::min(jper, 128);
 }
@@ -1998,7 +2009,8 @@ static int os_nks(int CinP, int wn, int64_t blocks, int cus, int step_channels) 
 // (choose_jper).  Where the lines lie:
 //   Up to 8 offsets: one block per CU.
 //   9 to 27 offsets: 96 columns at 40 % of the CUs (31k voxels, 243 blocks:
-// 25.9 us wide, 37.3 narrow; 110 blocks 23.9 / 24.8), 64 columns and wide
+// 25.9 us wide, 37.3 narrow; 110 blocks 23.9 / 24.8), at 60 % for less than
+// 96 channels (32 -> 96, 188 blocks 17.8 / 19.7), 64 columns and wide
 // inputs at half of them (128 -> 128, 243 blocks 32.4 / 37.2; 110 blocks 29.2
 // / 23.1), else at one block per CU (64 -> 128, 204 blocks 23.7 / 21.9).  A
 // second step down to 32 columns only where it fills the chip without a split
@@ -2006,7 +2018,8 @@ static int os_nks(int CinP, int wn, int64_t blocks, int cus, int step_channels) 
 // narrowing multiplies the gathered rows (256 -> 256, 32 row blocks: 53.0 us
 // at 32 columns, 34.8 at 64 and two splits).
 //   More offsets: split rather than narrow (125 offsets, 96 -> 96, 157 blocks
-// 101 -> 69 us), but for 128 columns of at most 64 channels, whose narrow
+// 101 -> 69 us), but for 96 columns of up to 16 channels (250 blocks 60.5 wide
+// and split, 52.3 narrow), for 128 columns of at most 64 channels, whose narrow
 // tiles pack two offsets per step (243 blocks 85 / 74), and of more channels
 // below a quarter of the CUs (55 blocks 48.6 / 43.4).
 //   Index-order layers of 256 columns and more whose 128-column blocks are
@@ -2019,9 +2032,9 @@ static int os_wn(int64_t num_targets, int c_out, int cus, int col_tile, int Kc, 
   const int64_t blocks = rows * div_up(cols, 32 * wn);
   const bool many = Kc > ring::kMapTileK, mid = Kc > 8 && !many;
   int64_t least = cus;
-  if (many) least = wn < 4 ? 0 : CinP <= 64 ? cus : cus / 4;
+  if (many) least = wn == 3 ? (CinP <= 16 ? cus : 0) : wn < 3 ? 0 : CinP <= 64 ? cus : cus / 4;
   else if (Kc > 8 && !ordered && c_out >= 256 && blocks > cus && 4 * blocks <= 5 * static_cast<int64_t>(cus)) return 3;
-  else if (mid && wn == 3) least = cus * 2 / 5;
+  else if (mid && wn == 3) least = CinP >= 96 ? cus * 2 / 5 : cus * 3 / 5;
   else if (mid && (wn == 2 || CinP >= 96)) least = cus / 2;
   if (wn == 1 || blocks >= least) return wn;
   if (wn == 3) return 1;

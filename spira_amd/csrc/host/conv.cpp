@@ -741,14 +741,19 @@ torch::Tensor forward_ws(int64_t S, int64_t T, int64_t gather_tile, int64_t scat
 // at d = 3.3 28.9 -> 29.9, at 5 101 -> 66, at 15 73 -> 35; 256 -> 256 at 3.3
 // 89 -> 127, at 5 352 -> 348, at 15 258 -> 157; outputs of 32 columns and
 // fewer are faster fused at every d (their atomics are few: 16 -> 16 at d = 15
-// 24 -> 34).  fp32's fused pass runs on the vector ALU: it wins only small
+// 24 -> 34).  Columns that the compacted kernel pads (48 to 64, 96 of wide
+// inputs to 128) want more pairs (96 -> 48 at d = 5 48 -> 60, 96 -> 96 80 ->
+// 89, at 12 142 -> 115; 125 offsets 32 -> 48 75 -> 93), and channels that need padded rows, a launch more,
+// 50k pairs in all (20 -> 48, 24k pairs 18 -> 22, 90k 40 -> 32).  fp32's fused pass runs on the vector ALU: it wins only small
 // layers (100M multiply-adds at 27 offsets 40 -> 43, 245M 86 -> 59, 800M 535 ->
 // 70; with 125 offsets 120M 48 -> 76, 390M 214 -> 186).
 static bool pairs_compact_pays(int64_t pairs, int64_t T, int64_t K, int64_t cin, int64_t cout, int dtype) {
   if (dtype == SPIRA_F32)
     return static_cast<double>(pairs) * cin * cout >= 1e8 * std::max(1.0, static_cast<double>(K) / 32);
   const double d = 64.0 * pairs / (static_cast<double>(std::max<int64_t>(T, 1)) * K);
-  return cout > 32 && d >= (cin > 128 ? 6.5 : 3.6);
+  const bool padded = cout % 64 != 0 && (cout < 64 || cin > 64);
+  if (cout <= 32 || (cout < 64 && K > 32) || (cin % 8 != 0 && pairs < 50000)) return false;
+  return d >= (cin > 128 || padded ? 6.5 : 3.6);
 }
 
 static void check_pairs(const torch::Tensor &naddrs, const torch::Tensor &qnaddrs, const torch::Tensor &nbmaps,

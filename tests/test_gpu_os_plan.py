@@ -17,9 +17,10 @@ from helpers import np_, rel_err
 #         T    K  cin cout  (column tile, splits)
 PLANS = [(400, 8, 32, 128, 64, 8), (16300, 27, 32, 32, 32, 2), (16500, 27, 32, 32, 32, 1),
          (12900, 27, 128, 128, 64, 1), (16500, 27, 128, 128, 128, 1), (7000, 27, 128, 128, 32, 1),
-         (12900, 27, 64, 96, 32, 1), (13000, 27, 64, 96, 96, 2), (20000, 27, 64, 256, 96, 1),
+         (19400, 27, 64, 96, 32, 1), (19600, 27, 64, 96, 96, 1),
+         (12900, 27, 96, 96, 32, 1), (13100, 27, 96, 96, 96, 1), (20000, 27, 64, 256, 96, 1),
          (20600, 27, 64, 256, 128, 1), (700, 125, 16, 16, 32, 42), (16300, 125, 16, 16, 32, 5),
-         (32600, 125, 32, 64, 64, 2), (32900, 125, 32, 64, 64, 1), (8000, 125, 96, 128, 64, 4),
+         (22800, 125, 32, 64, 64, 2), (23100, 125, 32, 64, 64, 1), (8000, 125, 96, 128, 64, 4),
          (8300, 125, 96, 128, 128, 7), (40900, 125, 96, 64, 64, 3), (41100, 125, 96, 64, 64, 1)]
 
 
