@@ -133,6 +133,19 @@ int spira_hip_downsample_chain(const void *keys, int64_t n, int key_bits, int le
                                void *const *out_keys, uint32_t *d_counts, uint32_t *d_unsorted, void *workspace,
                                size_t workspace_bytes, hipStream_t stream);
 
+/* Workspace bytes for spira_hip_downsample_grid. */
+int spira_hip_downsample_grid_workspace(int64_t n, int levels, size_t *bytes);
+
+/* spira_hip_downsample_chain by occupancy grids over the keys' bounding box:
+ * the same outputs for 1 to 8 levels of nested power-of-two strides (any
+ * ratio) and at least one key.  *d_flag (device, zeroed by the caller) gets
+ * bit 0 when the keys are not sorted ascending, and bit 1 when the box holds
+ * more cells than the workspace has bits, in which case the outputs are
+ * undefined and spira_hip_downsample_chain is the call. */
+int spira_hip_downsample_grid(const void *keys, int64_t n, int key_bits, int levels, const int32_t *strides,
+                              void *const *out_keys, uint32_t *d_counts, uint32_t *d_flag, void *workspace,
+                              size_t workspace_bytes, hipStream_t stream);
+
 /* ----------------------------------------------------------- kernel maps */
 
 #define SPIRA_KMAP_OS 0     /* [Tp, K] int32, column iz*O + o (z-major)            */

@@ -127,8 +127,8 @@ class KernelMapCache:
         # Map 0 (voxels[0] to voxels[0]) needs no downsampled level: it is
         # queued between the chained downsample and the host read of the
         # level counts, so that the GPU works on it while the host waits.
-        kmaps, outputs = [], None
-        launched = F.downsample_chain_launch(source_coordinates, target_strides) if kernel_sizes else None
+        kmaps, outputs, grid = [], None, True
+        launched = F.downsample_chain_launch(source_coordinates, target_strides, True) if kernel_sizes else None
         if launched is not None:
             levels, counts = launched
             host = torch.empty(counts.numel(), dtype=torch.int32, pin_memory=True)
@@ -140,8 +140,9 @@ class KernelMapCache:
             n = host.tolist()
             if n[-1] == 0:
                 outputs = [lv[:c] for lv, c in zip(levels, n[:-1])]
-        if outputs is None:  # strides that do not chain, or unsorted keys
-            outputs = F.streamed_output_generate(source_coordinates, target_strides)
+            grid = n[-1] & 2 == 0
+        if outputs is None:  # strides that do not chain, unsorted keys, or a box too wide for the grids
+            outputs = F.streamed_output_generate(source_coordinates, target_strides, grid)
         voxels = [source_coordinates] + list(outputs)
         self._coordinates_cache[s_stride] = voxels[0]
         for i, ts in enumerate(target_strides):

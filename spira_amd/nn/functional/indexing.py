@@ -52,21 +52,26 @@ def unflatten(coordinates: torch.Tensor) -> torch.Tensor:
     return _C.cuda_unflatten(coordinates)
 
 
-def streamed_output_generate(coordinates: torch.Tensor, target_strides: List[Tuple[int, int, int]]):
+def streamed_output_generate(coordinates: torch.Tensor, target_strides: List[Tuple[int, int, int]],
+                             grid: bool = True):
+    """``grid`` False: without the occupancy grids (a box known to be too wide)."""
     coordinates = coordinates.contiguous()
     _require_gpu(coordinates)
-    return _C.cuda_streamed_output_generate(coordinates, [as_tuple(s, size=3) for s in target_strides])
+    return _C.cuda_streamed_output_generate(coordinates, [as_tuple(s, size=3) for s in target_strides],
+                                              bool(grid))
 
 
-def downsample_chain_launch(coordinates: torch.Tensor, target_strides: List[Tuple[int, int, int]]):
+def downsample_chain_launch(coordinates: torch.Tensor, target_strides: List[Tuple[int, int, int]],
+                            grid: bool = False):
     """Queue the chained downsample of sorted keys on the current stream
     without reading anything back: ``(outputs, counts)``, the outputs at full
     capacity and ``counts`` a device int32 tensor of the level counts followed
     by the unsorted-input flag; ``None`` when the strides do not chain (or no
-    keys), for which :func:`streamed_output_generate` is the call."""
+    keys), for which :func:`streamed_output_generate` is the call.  ``grid``:
+    by occupancy grids; the flag is then 2 where the keys' box is too wide."""
     coordinates = coordinates.contiguous()
     _require_gpu(coordinates)
-    r = _C.cuda_downsample_chain_launch(coordinates, [as_tuple(s, size=3) for s in target_strides])
+    r = _C.cuda_downsample_chain_launch(coordinates, [as_tuple(s, size=3) for s in target_strides], bool(grid))
     if not r:
         return None
     return list(r[:-1]), r[-1]
