@@ -135,6 +135,7 @@ struct OrderEntry {
   uint32_t version = 0;
   int64_t T = 0;
   bool free = false;  // made with the map at no sorting cost (convert_transposed_os_ordered)
+                      // or sorted along with a network's other maps (prepare_row_orders)
   torch::Tensor order, masks, ordered_map;
   hipStream_t stream = nullptr;  // the stream the tensors were allocated and written on
 };
@@ -290,10 +291,22 @@ std::vector<torch::Tensor> prepare_row_order(const torch::Tensor &map, int64_t T
 // order and have none cached get it from one batched chain of launches
 // (spira_hip_kmap_row_order_batch: one sort over all maps' rows) when they
 // have 9 to 27 offsets, else one by one.  No reference counterpart.
+//
+// One sort over all rows costs little more than over the largest map's
+// alone, so a network's smaller 27-offset maps are ordered along with the
+// rest and their layers read the order (whole UNet pass, us, without -> with
+// the levels below 100k rows: indoor 200k voxels 2565 -> 2436, lidar 100k 2976
+// -> 2557).  Not below 12k rows (levels of 4k rows: no gain), and not where
+// the 27-offset maps together hold fewer than 150k rows (indoor 60k voxels,
+// 150k rows: 1800 -> 1769 to 1806; 20k voxels: 1560 -> 1618).
 void prepare_row_orders(const std::vector<torch::Tensor> &maps, const std::vector<int64_t> &Ts,
                         const std::vector<int64_t> &requests) {
   SPIRA_CHECK_ARG(maps.size() == Ts.size() && maps.size() == requests.size(),
                   "maps, target counts and requests must have the same length");
+  constexpr int64_t kTogether = 150000, kLeast = 12000;
+  int64_t rows = 0;
+  for (size_t i = 0; i < maps.size(); ++i)
+    if (requests[i] == -1 && maps[i].dim() == 2 && maps[i].size(1) == 27) rows += Ts[i];
   std::vector<size_t> batch;
   for (size_t i = 0; i < maps.size(); ++i) {
     const torch::Tensor &map = maps[i];
@@ -302,7 +315,8 @@ void prepare_row_orders(const std::vector<torch::Tensor> &maps, const std::vecto
     SPIRA_CHECK_ARG(map.size(0) >= Ts[i], "out_in_map has fewer rows than targets");
     SPIRA_CHECK_ARG(requests[i] >= -1 && requests[i] <= 1, "row order request must be -1, 0 or 1");
     const int64_t K = map.size(1);
-    if (!row_order_applies(Ts[i], K, static_cast<int>(requests[i])) || cached_order(map, Ts[i])) continue;
+    const bool along = row_order_enabled() && requests[i] == -1 && K == 27 && Ts[i] >= kLeast && rows >= kTogether;
+    if ((!along && !row_order_applies(Ts[i], K, static_cast<int>(requests[i]))) || cached_order(map, Ts[i])) continue;
     bool dup = false;  // (one map listed twice)
     for (size_t j : batch) dup |= maps[j].unsafeGetTensorImpl() == map.unsafeGetTensorImpl();
     if (dup) continue;
@@ -328,6 +342,7 @@ void prepare_row_orders(const std::vector<torch::Tensor> &maps, const std::vecto
       e.version = map._version();
       e.T = T;
       e.stream = current_stream();
+      e.free = requests[batch[b0 + q]] == -1;
       e.order = empty_i32({T}, map.device());
       e.masks = torch::empty({(T + 127) / 128 * 2}, torch::TensorOptions(map.device()).dtype(torch::kInt64));
       e.ordered_map = empty_i32({T, K}, map.device());

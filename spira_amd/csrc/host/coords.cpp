@@ -87,8 +87,8 @@ static bool chainable(const std::vector<Int3> &strides) {
 // strides do not chain or there are no keys (the caller then takes
 // streamed_output_generate).  With `grid` (up to 8 levels) by occupancy grids
 // (spira_hip_downsample_grid), whose flag has bit 1 set where the box of the
-// keys is too wide for them: 200k-voxel indoor scan, four levels, 158 us by
-// merging and 30 by grids.
+// keys is too wide for them: 200k-voxel indoor scan, four levels, 147 us by
+// merging and 32 by grids.
 std::vector<torch::Tensor> downsample_chain_launch(const torch::Tensor &keys, const std::vector<Int3> &strides,
                                                    bool grid) {
   SPIRA_CHECK_ARG(keys.dim() == 1, "coordinates should be already flattened");

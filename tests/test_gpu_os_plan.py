@@ -53,3 +53,25 @@ def test_output(dev, T, K, cin, cout, tile, splits):
     if cin > 32 and cin % 32 == 0:
         y2 = F.sparse_convolution_forward_os(S, T, m, X[:, :32].contiguous(), W, sources2=X[:, 32:].contiguous())
         assert rel_err(np_(y2[rows].float()), np_(ref)) <= 4e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [(70000, 80000, 20000, 12000, 11999), (149000, 999), (12000,) * 13])
+def test_orders_made_together(dev, sizes):
+    """A network's 27-offset maps ordered by one batch, on both sides of its
+    lines (150k rows together, 12k rows each): every layer equals the one
+    that is told to take no order, in fp16 and float32, with and without a
+    split of the offsets."""
+    g = torch.Generator().manual_seed(len(sizes))
+    maps = []
+    for T in sizes:
+        m = torch.randint(-1000, 1000, (T, 27), generator=g, dtype=torch.int32).clamp_(min=-1)
+        maps.append(torch.nn.functional.pad(m, (0, 0, 0, -T % 128), value=-1).to(dev))
+    F.prepare_row_orders(maps, list(sizes), [-1] * len(sizes))
+    for m, T in zip(maps[-3:], sizes[-3:]):
+        for cin, cout, dtype in ((32, 32, torch.float16), (64, 256, torch.float16), (32, 32, torch.float32)):
+            X = torch.randn(1000, cin, generator=g).to(dtype).to(dev)
+            W = (torch.randn(27, cin, cout, generator=g) / np.sqrt(9 * cin)).to(dtype).to(dev)
+            y = F.sparse_convolution_forward_os(1000, T, m, X, W)
+            y0 = F.sparse_convolution_forward_os(1000, T, m, X, W, tuning=(0, 0, 0, 0, 0, 0))
+            assert rel_err(np_(y.float()), np_(y0.float())) <= (4e-3 if dtype == torch.float16 else 1e-5)
