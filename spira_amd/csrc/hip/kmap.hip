@@ -28,6 +28,7 @@
 //     writes it out contiguously.
 
 #include "common.hpp"
+#include "radix.hpp"
 #include "../../../include/spira_hip.h"
 
 #include <rocprim/rocprim.hpp>
@@ -1339,7 +1340,7 @@ static RowBatchParts row_batch_parts(int64_t N, int64_t G, int nmaps, void *base
                                   static_cast<uint64_t *>(nullptr), static_cast<const int32_t *>(nullptr),
                                   static_cast<int32_t *>(nullptr), static_cast<size_t>(N), 0, hi);
   RowBatchParts r{};
-  r.tmp_bytes = b;
+  r.tmp_bytes = std::max(b, sort_bits_bytes(N));
   char *p = static_cast<char *>(base);
   size_t off = 0;
   auto take = [&](size_t bytes) {
@@ -1670,11 +1671,19 @@ int spira_hip_kmap_row_order_batch(int n, const spira_hip_row_order_job_t *jobs,
                      256 * kmax * sizeof(int32_t), stream, bt, w.keys, w.iota);
   SPIRA_HIP_LAUNCH_CHECK();
   const int hi = 32 + (n > 1 ? 32 - __builtin_clz(static_cast<unsigned>(n - 1)) : 0);
-  // (rocPRIM: at 438k keys of 34 bits it measured ahead of radix.hip's sort,
-  // config-4 step 2.418 against 2.434 ms)
-  size_t tb = w.tmp_bytes;
-  SPIRA_HIP_TRY(rocprim::radix_sort_pairs(w.tmp, tb, w.keys, w.keys_out, w.iota, w.sorted, static_cast<size_t>(N), 0,
-                                          hi, stream));
+  // (up to kSortBitsMost rows; above, every placing block's read of all
+  // tiles' counts costs more than rocPRIM's sort)
+  if (N <= kSortBitsMost) {
+    uint64_t *keys[2] = {w.keys, w.keys_out};
+    int32_t *vals[2] = {w.iota, w.sorted};
+    if (int rs = sort_bits(keys, vals, N, hi, w.tmp, w.tmp_bytes, stream)) return rs;
+    w.keys_out = keys[0];
+    w.sorted = vals[0];
+  } else {
+    size_t tb = w.tmp_bytes;
+    SPIRA_HIP_TRY(rocprim::radix_sort_pairs(w.tmp, tb, w.keys, w.keys_out, w.iota, w.sorted, static_cast<size_t>(N),
+                                            0, hi, stream));
+  }
   hipLaunchKernelGGL(group_union_batch_kernel, dim3(static_cast<unsigned>(bt.group_blk[n])), dim3(256), 0, stream, bt,
                      w.keys_out, w.gm, w.gkey);
   SPIRA_HIP_LAUNCH_CHECK();

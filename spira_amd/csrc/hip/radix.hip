@@ -38,10 +38,14 @@
 // ~4 us ranking (with the key loads), ~5 us look-back and ~3.5 us staged
 // scatter; the look-back's device-coherent loads grow with tiles x digits,
 // and each exchange between blocks costs a device-scope round trip of
-// ~1.5 us.  flatten_sort and the row order therefore keep rocPRIM.
+// ~1.5 us.  flatten_sort and a single map's row order therefore keep rocPRIM;
+// the batched row orders, whose bits the host knows, take sort_bits below.
 #include "common.hpp"
 #include "radix.hpp"
 #include "../../../include/spira_hip.h"
+
+#include <algorithm>
+#include <utility>
 
 namespace spira_hip {
 
@@ -345,6 +349,181 @@ __global__ __launch_bounds__(kThreads) void sk_pass_kernel(int pass, int64_t n, 
   }
 }
 
+// ---------------------------------------------------------------------------
+// Sort over known low bits without a look-back: per digit (9 bits at most) a
+// launch that counts every 2048-key tile's digits and one that places them.
+// A placing block reads all tiles' counts itself (16-bit, 1 KB per tile, eight
+// tiles per round of its eight waves) for its digits' global bases, so no
+// block waits for another.  Bound by the launches and, within one, by the
+// chain of loads, ranks and scans; the counts read grow with the square of
+// the keys, which sets kSortBitsMost.
+// Measured on the rows of a UNet's four larger maps (438k keys of 34 bits, four
+// digits): 79 us, 4.5 counting and 15 placing per digit; rocPRIM's merge sort,
+// which it takes for such sizes, 132 us.
+// ---------------------------------------------------------------------------
+constexpr int kSmallItems = 4;
+constexpr int kSmallTile = kThreads * kSmallItems;
+
+template <typename CT>
+__global__ __launch_bounds__(kThreads) void sk_count_kernel(const CT *__restrict__ keys, int64_t n, int shift,
+                                                            int width, uint16_t *__restrict__ counts) {
+  __shared__ uint32_t h[kMaxBins];
+  const int tid = threadIdx.x;
+  h[tid] = 0;
+  __syncthreads();
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * kSmallTile;
+  CT k[kSmallItems];
+#pragma unroll
+  for (int j = 0; j < kSmallItems; ++j) k[j] = keys[min(base + j * kThreads + tid, n - 1)];
+#pragma unroll
+  for (int j = 0; j < kSmallItems; ++j) {
+    const bool ok = base + j * kThreads + tid < n;
+    const uint32_t d = digit(k[j], shift, width);
+    // (a digit shared by the whole wave is one LDS add)
+    const uint32_t d0 = __builtin_amdgcn_readfirstlane(d);
+    const uint64_t valid = __ballot(ok);
+    if (__ballot(d != d0) == 0) {
+      if ((tid & 63) == 0) atomicAdd(&h[d0], static_cast<uint32_t>(__builtin_popcountll(valid)));
+    } else if (ok) {
+      atomicAdd(&h[d], 1u);
+    }
+  }
+  __syncthreads();
+  counts[static_cast<int64_t>(blockIdx.x) * kMaxBins + tid] = static_cast<uint16_t>(h[tid]);
+}
+
+template <typename CT>
+__global__ __launch_bounds__(kThreads) void sk_place_kernel(const CT *__restrict__ kin,
+                                                            const int32_t *__restrict__ vin, CT *__restrict__ kout,
+                                                            int32_t *__restrict__ vout, int64_t n, int ntiles,
+                                                            int shift, int width,
+                                                            const uint16_t *__restrict__ counts) {
+  __shared__ uint16_t wcnt[kWaves][kMaxBins];  // per-wave running counts, then wave prefixes
+  __shared__ uint32_t toff[kMaxBins], gpos[kMaxBins], wsum[2][kWaves];
+  struct Sums {
+    uint32_t tot[kWaves][kMaxBins], pre[kWaves][kMaxBins];
+  };
+  struct Stage {
+    CT key[kSmallTile];
+    int32_t val[kSmallTile];
+  };
+  __shared__ __align__(16) union {  // (the sums are read before the tile is staged)
+    Sums sums;
+    Stage stage;
+  } u;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, tile = blockIdx.x;
+  const int64_t tbase = static_cast<int64_t>(tile) * kSmallTile;
+  const int64_t wbase = tbase + wave * (64 * kSmallItems);
+  CT key[kSmallItems];
+  int32_t val[kSmallItems];
+#pragma unroll
+  for (int j = 0; j < kSmallItems; ++j) {
+    const int64_t i = min(wbase + j * 64 + lane, n - 1);
+    key[j] = kin[i];
+    val[j] = vin[i];
+  }
+  for (int i = lane; i < kMaxBins / 2; i += 64) reinterpret_cast<uint32_t *>(&wcnt[wave][0])[i] = 0;
+  // the counts of digits 8 lane .. 8 lane + 7 in all tiles and in those before
+  {
+    uint32_t tot[8] = {}, pre[8] = {};
+    const uint4 *c4 = reinterpret_cast<const uint4 *>(counts) + lane;
+#pragma unroll 8
+    for (int t = wave; t < ntiles; t += kWaves) {
+      const uint4 q = c4[t * (kMaxBins / 8)];
+      const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t lo = w[e] & 0xFFFFu, hi = w[e] >> 16;
+        tot[2 * e] += lo;
+        tot[2 * e + 1] += hi;
+        pre[2 * e] += t < tile ? lo : 0u;
+        pre[2 * e + 1] += t < tile ? hi : 0u;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e += 4) {
+      *reinterpret_cast<uint4 *>(&u.sums.tot[wave][lane * 8 + e]) = uint4{tot[e], tot[e + 1], tot[e + 2], tot[e + 3]};
+      *reinterpret_cast<uint4 *>(&u.sums.pre[wave][lane * 8 + e]) = uint4{pre[e], pre[e + 1], pre[e + 2], pre[e + 3]};
+    }
+  }
+  // stable ranks among the wave's keys, in rounds of 64
+  uint32_t rank[kSmallItems];
+  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int j = 0; j < kSmallItems; ++j) {
+    const bool ok = wbase + j * 64 + lane < n;
+    const uint32_t d = digit(key[j], shift, width);
+    uint64_t peers = __ballot(ok);
+    for (int bit = 0; bit < width; ++bit) {
+      const bool on = (d >> bit) & 1u;
+      const uint64_t mb = __ballot(on);
+      peers &= on ? mb : ~mb;
+    }
+    const uint32_t before = wcnt[wave][d];
+    rank[j] = before + static_cast<uint32_t>(__builtin_popcountll(peers & lt));
+    __builtin_amdgcn_wave_barrier();
+    if (ok && (peers & lt) == 0) wcnt[wave][d] = static_cast<uint16_t>(before + __builtin_popcountll(peers));
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+  // thread t: digit t
+  uint32_t cnt = 0, tot = 0, pre = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    const uint32_t v = wcnt[w][tid];
+    wcnt[w][tid] = static_cast<uint16_t>(cnt);
+    cnt += v;
+    tot += u.sums.tot[w][tid];
+    pre += u.sums.pre[w][tid];
+  }
+  uint32_t ti = tot, ci = cnt;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t a = __shfl_up(ti, o, 64), b = __shfl_up(ci, o, 64);
+    if (lane >= o) {
+      ti += a;
+      ci += b;
+    }
+  }
+  if (lane == 63) {
+    wsum[0][wave] = ti;
+    wsum[1][wave] = ci;
+  }
+  __syncthreads();
+  uint32_t gbase = ti - tot, off = ci - cnt;
+  for (int w = 0; w < wave; ++w) {
+    gbase += wsum[0][w];
+    off += wsum[1][w];
+  }
+  toff[tid] = off;
+  gpos[tid] = gbase + pre;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kSmallItems; ++j) {
+    if (wbase + j * 64 + lane < n) {
+      const uint32_t d = digit(key[j], shift, width);
+      const uint32_t l = toff[d] + wcnt[wave][d] + rank[j];
+      u.stage.key[l] = key[j];
+      u.stage.val[l] = val[j];
+    }
+  }
+  __syncthreads();
+  const int here = static_cast<int>(n - tbase < kSmallTile ? n - tbase : kSmallTile);
+#pragma unroll
+  for (int j = 0; j < kSmallItems; ++j) {
+    const int l = j * kThreads + tid;
+    if (l < here) {
+      const CT k = u.stage.key[l];
+      const uint32_t d = digit(k, shift, width);
+      const uint32_t pos = gpos[d] + (static_cast<uint32_t>(l) - toff[d]);
+      kout[pos] = k;
+      vout[pos] = u.stage.val[l];
+    }
+  }
+}
+
 static inline size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
 struct Parts {
@@ -420,6 +599,32 @@ template <typename CT> int sort_status(const void *ws, int64_t n, bool with_valu
   SPIRA_HIP_TRY(hipMemcpyAsync(&stalled, &w.plan->stalled, sizeof(stalled), hipMemcpyDeviceToHost, s));
   SPIRA_HIP_TRY(hipStreamSynchronize(s));
   SPIRA_HIP_REQUIRE(stalled == 0, "radix_sort: a look-back wait ran out; the output is incomplete");
+  return kOk;
+}
+
+size_t sort_bits_bytes(int64_t n) {
+  return static_cast<size_t>(div_up(std::max<int64_t>(n, 1), sortk::kSmallTile)) * sortk::kMaxBins * 2;
+}
+
+int sort_bits(uint64_t *(&keys)[2], int32_t *(&vals)[2], int64_t n, int bits, void *ws, size_t ws_bytes,
+              hipStream_t s) {
+  using namespace sortk;
+  SPIRA_HIP_REQUIRE(n >= 1 && n <= kSortBitsMost && bits >= 1 && bits <= 64, "sort_bits: size out of range");
+  SPIRA_HIP_REQUIRE(ws != nullptr && ws_bytes >= sort_bits_bytes(n), "sort_bits: workspace too small");
+  const int ntiles = static_cast<int>(div_up(n, kSmallTile));
+  uint16_t *counts = static_cast<uint16_t *>(ws);
+  const int passes = static_cast<int>(div_up(bits, kMaxWidth));
+  for (int p = 0, shift = 0; p < passes; ++p) {
+    const int width = static_cast<int>(div_up(bits - shift, passes - p));
+    hipLaunchKernelGGL(sk_count_kernel<uint64_t>, dim3(ntiles), dim3(kThreads), 0, s, keys[0], n, shift, width,
+                       counts);
+    hipLaunchKernelGGL(sk_place_kernel<uint64_t>, dim3(ntiles), dim3(kThreads), 0, s, keys[0], vals[0], keys[1],
+                       vals[1], n, ntiles, shift, width, counts);
+    std::swap(keys[0], keys[1]);
+    std::swap(vals[0], vals[1]);
+    shift += width;
+  }
+  SPIRA_HIP_LAUNCH_CHECK();
   return kOk;
 }
 

@@ -24,4 +24,13 @@ int sort_keys_values(const CT *keys_in, const int32_t *vals_in, CT *keys_out, in
 // look-back wait run out (its output is then incomplete).
 template <typename CT> int sort_status(const void *ws, int64_t n, bool with_values, hipStream_t s);
 
+// Stable ascending sort of n keys by their low `bits` bits (the others zero),
+// the values following, between the two buffers of each: keys[0] / vals[0]
+// hold the input and, on return, name the buffers of the output.  No block
+// waits for another and no memory is set, so that it can be captured.
+constexpr int64_t kSortBitsMost = 700000;
+size_t sort_bits_bytes(int64_t n);
+int sort_bits(uint64_t *(&keys)[2], int32_t *(&vals)[2], int64_t n, int bits, void *ws, size_t ws_bytes,
+              hipStream_t s);
+
 }  // namespace spira_hip
