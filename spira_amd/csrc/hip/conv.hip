@@ -2118,6 +2118,11 @@ static OsPlan plan_os(int64_t T, int Kc, int Cin, int CinP, bool cat, int Cout, 
   pl.aligned = Cin % 8 == 0;
   pl.xcd = tn.block_order;
   pl.nks = pl.aligned ? os_nks(CinP, pl.wn, pl.gx * pl.gy * pl.splits, cus, tn.step_channels) : 2;
+  // pointwise layers stream their rows: steps of at most 64 channels, whose
+  // smaller ring leaves room for more blocks per CU (200k rows, 128 -> 96
+  // 34.9 -> 24.4 us, 96 -> 96 33.0 -> 22.5, 128 -> 64 25.1 -> 23.7; 64-channel steps
+  // are what wider tiles take anyway)
+  if (!has_map && pl.nks == 8 && tn.step_channels == 0) pl.nks = 4;
   pl.pack = 1;
   // offset packing: 16- and 32-channel inputs of kernels with more than 27
   // offsets (map entries fetched per step) run four offsets per step (64-

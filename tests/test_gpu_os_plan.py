@@ -75,3 +75,18 @@ def test_orders_made_together(dev, sizes):
             y = F.sparse_convolution_forward_os(1000, T, m, X, W)
             y0 = F.sparse_convolution_forward_os(1000, T, m, X, W, tuning=(0, 0, 0, 0, 0, 0))
             assert rel_err(np_(y.float()), np_(y0.float())) <= (4e-3 if dtype == torch.float16 else 1e-5)
+
+
+@pytest.mark.parametrize("T,cin,cout", [(1, 128, 96), (129, 96, 96), (4097, 128, 64), (70001, 112, 96)])
+def test_pointwise_plan(T, cin, cout):
+    assert _native._C.conv_os_plan(T, 1, cin, 0, cout, False)[1] <= 64
+    assert _native._C.conv_os_plan(T, 1, cin, 0, cout, False, (0, 128, 0, 0, 0, -1))[1] == 128
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,cin,cout", [(1, 128, 96), (129, 96, 96), (4097, 128, 64), (70001, 112, 96)])
+def test_pointwise_output(dev, T, cin, cout):
+    g = torch.Generator().manual_seed(T)
+    X = torch.randn(T, cin, generator=g).half().to(dev)
+    W = (torch.randn(1, cin, cout, generator=g) / np.sqrt(cin)).half().to(dev)
+    assert rel_err(np_(F.dense_forward(X, W).float()), np_(X.double() @ W[0].double())) <= 4e-3
