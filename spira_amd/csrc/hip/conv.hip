@@ -1876,12 +1876,10 @@ static inline int bm_for(int wn) {
 // nearly every CU has one (48 -> 16, 250 blocks: 18.8 us with two, 20.9 with
 // one).
 //   More offsets: a block runs over a hundred dependent steps, so they split
-// until two blocks share a CU (2.5 of 32 columns), at most into eighths, and
-// inputs of 96 channels and more into thirds up to 1.25 blocks per CU.  125
-// offsets, 20k voxels, 157 row tiles: 64 -> 64 57 -> 41 us, 96 -> 96 101 ->
-// 69, 128 -> 128 120 -> 93, 16 -> 16 30 -> 22; 128 -> 128 at 263 row tiles
-// 190 -> 160.  Not wide tiles of up to 32 channels on 70 % of the CUs, which
-// pack four offsets per step unsplit (16 -> 64, 250 blocks 48.0 / 42.2).
+// until two blocks share a CU (2.5 of 32 columns), at most into eighths
+// (plan_os takes three parts and more back where two at most are due).  Not
+// wide tiles of up to 32 channels on 70 % of the CUs, which pack four offsets
+// per step unsplit (16 -> 64, 250 blocks 48.0 / 42.2).
 static int choose_jper(int64_t blocks_xy, int Kc, int CinP, int wn, int cus, int splits = 0) {
   int jper = Kc;
   int64_t n = 1;
@@ -1891,7 +1889,6 @@ static int choose_jper(int64_t blocks_xy, int Kc, int CinP, int wn, int cus, int
     const int64_t most = std::max<int64_t>(CinP >= 64 && wn == 2 ? 6 : 8, cus / blocks_xy);
     if (CinP <= 32 && wn >= 2 && blocks_xy * 10 > static_cast<int64_t>(cus) * 7) n = 1;
     else if (blocks_xy < cus) n = std::min<int64_t>((wn == 1 && CinP <= 32 ? 5 : 4) * cus / (2 * blocks_xy), most);
-    else if (CinP >= 96 && 4 * blocks_xy <= 5 * static_cast<int64_t>(cus)) n = 3;
   } else if (Kc > 1 && blocks_xy < cus) {
     const bool deep = CinP >= 256 || (CinP > 16 && CinP % 32 != 0);
     const int64_t limit = deep ? (wn == 1 ? cus : cus * 3 / 5) : wn == 3 ? cus * 2 / 5 : cus / 2;
@@ -2042,6 +2039,13 @@ static int os_wn(int64_t num_targets, int c_out, int cus, int col_tile, int Kc, 
   return wn == 4 && mid && 2 * half < cus && 10 * half >= 3 * static_cast<int64_t>(cus) ? 1 : wn / 2;
 }
 
+// The widest tile, narrowed once where its grid holds less than a block per CU.
+static int narrowed_wn(int64_t num_targets, int c_out, int cus) {
+  const int wn = wn_for(c_out);
+  const int64_t blocks = div_up(num_targets, bm_for(1)) * div_up(pad_out(c_out), 32 * wn);
+  return wn == 1 || blocks >= cus ? wn : wn == 3 ? 1 : wn / 2;
+}
+
 // A third ring stage (two steps of gathers in flight instead of one) for
 // 64-channel steps of 96- and 128-column tiles and for 128-channel steps of
 // 32- and 64-column tiles, where the grid, at the larger block's LDS, still
@@ -2115,6 +2119,27 @@ static OsPlan plan_os(int64_t T, int Kc, int Cin, int CinP, bool cat, int Cout, 
   // small layers split their offsets over grid z
   pl.jper = choose_jper(pl.gx * pl.gy, Kc, CinP, pl.wn, cus, tn.offset_splits);
   pl.splits = static_cast<int>(div_up(Kc, pl.jper));
+  // Parts add to zeros by atomics: two give one sum in either order, three or
+  // more a sum that changes from run to run, and any other number of parts
+  // other last bits.  So where the narrowed grid holds half a block per CU, a
+  // layer is split as that grid asks, once or not at all: the kernels of more
+  // than 27 offsets exactly so, the others at most.  (What it costs: four
+  // levels of 125-offset layers, 30k to 17k voxels, 1.50 ms; in up to three
+  // parts 1.25 ms, with outputs that differ by 4e-4 between two runs.)
+  if (tn.offset_splits == 0) {
+    const int wn = tn.col_tile ? pl.wn : narrowed_wn(T, Cout, cus);
+    const int64_t gx = div_up(T, bm_for(wn)), gy = div_up(pad_out(Cout), 32 * wn);
+    const int jper = static_cast<int>(std::min<int64_t>(gx * gy < cus ? div_up(Kc, 2) : Kc, 128));
+    const int parts = static_cast<int>(div_up(Kc, jper));
+    if (2 * gx * gy >= cus && parts <= 2 && (Kc > ring::kMapTileK ? pl.splits != parts : pl.splits > 2)) {
+      pl.wn = wn;
+      pl.bm = bm_for(wn);
+      pl.gx = gx;
+      pl.gy = gy;
+      pl.jper = jper;
+      pl.splits = parts;
+    }
+  }
   pl.aligned = Cin % 8 == 0;
   pl.xcd = tn.block_order;
   pl.nks = pl.aligned ? os_nks(CinP, pl.wn, pl.gx * pl.gy * pl.splits, cus, tn.step_channels) : 2;

@@ -5,6 +5,8 @@ output against a float64 sum over the map.
 Tolerance, max |error| / RMS(reference): the fp16 store rounds to 2^-11 of a
 value that may be 6 x RMS (3e-3), and the fp32 sums of the splits add far less
 -> 4e-3."""
+import itertools
+
 import numpy as np
 import pytest
 import torch
@@ -19,9 +21,10 @@ PLANS = [(400, 8, 32, 128, 64, 8), (16300, 27, 32, 32, 32, 2), (16500, 27, 32, 3
          (12900, 27, 128, 128, 64, 1), (16500, 27, 128, 128, 128, 1), (7000, 27, 128, 128, 32, 1),
          (19400, 27, 64, 96, 32, 1), (19600, 27, 64, 96, 96, 1),
          (12900, 27, 96, 96, 32, 1), (13100, 27, 96, 96, 96, 1), (20000, 27, 64, 256, 96, 1),
-         (20600, 27, 64, 256, 128, 1), (700, 125, 16, 16, 32, 42), (16300, 125, 16, 16, 32, 5),
-         (22800, 125, 32, 64, 64, 2), (23100, 125, 32, 64, 64, 1), (8000, 125, 96, 128, 64, 4),
-         (8300, 125, 96, 128, 128, 7), (40900, 125, 96, 64, 64, 3), (41100, 125, 96, 64, 64, 1)]
+         (20600, 27, 64, 256, 128, 1), (700, 125, 16, 16, 32, 42), (16200, 125, 16, 16, 32, 5),
+         (16300, 125, 16, 16, 32, 2),
+         (22800, 125, 32, 64, 32, 1), (23100, 125, 32, 64, 64, 1), (8000, 125, 96, 128, 64, 4),
+         (8300, 125, 96, 128, 64, 2), (17212, 125, 128, 128, 64, 1), (40900, 125, 96, 64, 64, 1)]
 
 
 @pytest.mark.parametrize("T,K,cin,cout,tile,splits", PLANS)
@@ -30,6 +33,22 @@ def test_plan(T, K, cin, cout, tile, splits):
         pytest.skip("the lines are stated for 256 CUs")
     plan = _native._C.conv_os_plan(T, K, cin, 0, cout, True)
     assert (plan[0], plan[2]) == (tile, splits)
+
+
+@pytest.mark.parametrize("K", [8, 27, 28, 64, 125])
+def test_parts_of_grids_of_half_the_chip(K):
+    """Three parts or more add in no fixed order: none where the grid, its
+    tile narrowed once, holds half a block per CU or more; there a kernel of
+    more than 27 offsets is split in two below one block per CU, else not."""
+    for rows, cin, cout in itertools.product((1, 5, 31, 33, 42, 43, 63, 65, 127, 128, 135, 158, 255, 257, 319),
+                                             (8, 16, 32, 48, 64, 96, 128, 256), (16, 32, 48, 64, 96, 128, 256, 384)):
+        plan = _native._C.conv_os_plan(128 * rows, K, cin, 0, cout, True)
+        wide = 32 * min(4, -(-cout // 32))
+        narrow = wide if wide == 32 or rows * -(-cout // wide) >= 256 else 32 if wide == 96 else wide // 2
+        if rows * -(-cout // narrow) >= 128:
+            assert plan[2] <= 2, (rows, cin, cout, plan)
+            if K > 27:
+                assert plan[2] == (2 if rows * -(-cout // narrow) < 256 else 1), (rows, cin, cout, plan)
 
 
 @pytest.mark.gpu
@@ -49,6 +68,9 @@ def test_output(dev, T, K, cin, cout, tile, splits):
     for k in range(K):
         ref += Xz[m[rows, k].long()] @ W[k].double()
     assert rel_err(np_(y[rows].float()), np_(ref)) <= 4e-3
+    if splits <= 2:  # one sum on every call
+        for _ in range(3):
+            assert torch.equal(y, F.sparse_convolution_forward_os(S, T, m, X, W))
     # a concatenated input plans by the channels of both parts
     if cin > 32 and cin % 32 == 0:
         y2 = F.sparse_convolution_forward_os(S, T, m, X[:, :32].contiguous(), W, sources2=X[:, 32:].contiguous())
