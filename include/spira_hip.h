@@ -382,16 +382,17 @@ typedef struct {
  * its offsets over blocks, or, under work balance (balance_offsets), a work
  * list and fp32 partial tiles.  The workspace must be zero-filled before its
  * first use; every call leaves it zero-filled, so a caller keeps one buffer
- * per stream (calls that overlap on one buffer race). */
+ * per stream (calls that overlap on one buffer race).  Enough for both forms of
+ * the map (index or row order) and for a concatenation of any second part. */
 int spira_hip_conv_os_workspace(int64_t num_targets, int num_offsets, int c_in, int c_out, int dtype, int out_mode,
                                 const spira_hip_os_tuning_t *tuning, size_t *bytes);
 
 /* The launch spira_hip_conv_os would make for a layer (c_in2 > 0: the
- * concatenated form; has_map 0: the identity map) under `tuning`: plan[0..5]
- * = column tile (output channels), step channels, offset splits, kernel
- * offsets per step, grid x, grid y.  Runs on the host only.  (No reference
- * counterpart: it lets a caller or a test see what a tuning changes.)  plan[6]
- * = block order. */
+ * concatenated form; has_map 0: the identity map, 1: a map in index order, 2:
+ * one in row order with group masks) under `tuning`: plan[0..6] = column tile
+ * (output channels), step channels, offset splits, kernel offsets per step,
+ * grid x, grid y, block order.  Runs on the host only.  (No reference
+ * counterpart: it lets a caller or a test see what a tuning changes.) */
 int spira_hip_conv_os_plan(int64_t num_targets, int num_offsets, int c_in, int c_in2, int c_out, int has_map,
                            int out_mode, const spira_hip_os_tuning_t *tuning, int32_t *plan);
 

@@ -2339,17 +2339,31 @@ int spira_hip_prepare_weights(const void *weights, int num_offsets, int c_in, in
 
 int spira_hip_conv_os_workspace(int64_t num_targets, int num_offsets, int c_in, int c_out, int dtype, int out_mode,
                                 const spira_hip_os_tuning_t *tuning, size_t *bytes) {
+  (void)c_in;
   *bytes = 0;
   const spira_hip_os_tuning_t tn = tuning_of(tuning);
   if (int rc = check_tuning(tn)) return rc;
   if (!mfma_path(dtype) || out_mode != SPIRA_OUT_STORE || num_targets <= 0) return kOk;
-  const OsPlan pl = plan_os(num_targets, num_offsets, c_in, pad_in(c_in), false, c_out, true, true, tn);
-  // (a concatenation's plan goes by the channels of both parts, of which c_in
-  // may name the first alone: splits of the widest input count too)
-  const OsPlan wide = plan_os(num_targets, num_offsets, 512, 512, false, c_out, true, true, tn);
-  if (pl.splits > 1 || wide.splits > 1)
+  // Whatever the launch may plan: the query knows neither the row order nor
+  // a concatenation's second part.  Offsets are split on grids of less than a
+  // block per CU, at its fewest with the widest tile, or past 128 offsets.
+  const int wn = tn.col_tile ? tn.col_tile / 32 : wn_for(c_out);
+  const int64_t gx = div_up(num_targets, bm_for(wn)), cols = pad_out(c_out);
+  const bool few = gx * div_up(cols, 32 * wn) < device_cu_count();
+  if (tn.offset_splits > 1 || num_offsets > 128 || (tn.offset_splits == 0 && num_offsets > 1 && few))
     *bytes = static_cast<size_t>(num_targets) * c_out * sizeof(float);
-  *bytes = std::max(*bytes, pl.bal_bytes());
+  // (work balance: the tile that pads its columns most)
+  if (tn.balance_offsets > 0 && num_offsets <= 128) {
+    OsPlan pl{};
+    pl.bal = tn.balance_offsets;
+    pl.zmax = static_cast<int>(std::min<int64_t>(8, div_up(num_offsets, tn.balance_offsets)));
+    for (pl.wn = tn.col_tile ? wn : 1; pl.wn <= (tn.col_tile ? wn : 4); ++pl.wn) {
+      pl.bm = bm_for(pl.wn);
+      pl.gx = div_up(num_targets, pl.bm);
+      pl.gy = div_up(cols, 32 * pl.wn);
+      *bytes = std::max(*bytes, pl.bal_bytes());
+    }
+  }
   return kOk;
 }
 
@@ -2361,7 +2375,7 @@ int spira_hip_conv_os_plan(int64_t num_targets, int num_offsets, int c_in, int c
                     "conv_os_plan: empty layer or no output array");
   const int cin_all = c_in + c_in2;
   const OsPlan pl = plan_os(num_targets, num_offsets, cin_all, pad_in(cin_all), c_in2 > 0, c_out, has_map != 0,
-                            out_mode == SPIRA_OUT_STORE, tn);
+                            out_mode == SPIRA_OUT_STORE, tn, has_map == 2);
   plan[0] = pl.wn * 32;
   plan[1] = pl.nks * 16;
   plan[2] = pl.splits;

@@ -516,11 +516,8 @@ static void run_os(const torch::Tensor *map, int64_t S, int64_t T, const torch::
   const bool walk = tn.k.row_walk == 1 && map && dtype == SPIRA_F16 && !X2 && W.size(1) <= 16 &&
                     mode == SPIRA_OUT_STORE && K <= 128;
   auto P = prepared_weights(W);
-  size_t wsb = 0;
   const int64_t cin_run =
       (!split && dtype == SPIRA_F16 && W.size(1) % 8 != 0) ? (W.size(1) + 7) / 8 * 8 : W.size(1);
-  check_rc(spira_hip_conv_os_workspace(T, K, cin_run, W.size(2), dtype, mode, &tn.k, &wsb), "conv_os");
-  auto ws = zeroed_workspace(wsb, dev);
   const int32_t *order = nullptr;
   const uint64_t *masks = nullptr;
   if (map && dtype == SPIRA_F16 && !walk) {
@@ -540,6 +537,17 @@ static void run_os(const torch::Tensor *map, int64_t S, int64_t T, const torch::
       mp = oe->ordered_map.data_ptr<int32_t>();
     }
   }
+  size_t wsb = 0;
+  if (dtype == SPIRA_F16 && mode == SPIRA_OUT_STORE && T > 0) {
+    // (the query covers every form of the layer; most need nothing)
+    int32_t plan[7];
+    check_rc(spira_hip_conv_os_plan(T, K, split ? X.size(1) : cin_run, split ? X2->size(1) : 0, W.size(2),
+                                    mp ? (masks ? 2 : 1) : 0, mode, &tn.k, plan),
+             "conv_os");
+    if (plan[2] > 1 || tn.k.balance_offsets > 0)
+      check_rc(spira_hip_conv_os_workspace(T, K, cin_run, W.size(2), dtype, mode, &tn.k, &wsb), "conv_os");
+  }
+  auto ws = zeroed_workspace(wsb, dev);
   // fp16 rows whose width is not a multiple of 8 channels (the 3-channel
   // stem) are padded with zero channels to 16-byte rows, which the MMA
   // kernel gathers with one vector load each; the prepared weights already
@@ -1000,12 +1008,12 @@ float time_conv_os(int64_t S, int64_t T, const std::optional<torch::Tensor> &out
 // (col_tile, step_channels, offset_splits, offsets_per_step, grid_x, grid_y,
 // block_order).
 // No reference counterpart: it shows what a layer's tuning changes.
-std::vector<int64_t> conv_os_plan(int64_t T, int64_t K, int64_t cin, int64_t cin2, int64_t cout, bool has_map,
+std::vector<int64_t> conv_os_plan(int64_t T, int64_t K, int64_t cin, int64_t cin2, int64_t cout, int64_t has_map,
                                   const TuneArg &tuning) {
   const OsTune tn = tune_of(tuning);
   int32_t plan[7] = {};
   check_rc(spira_hip_conv_os_plan(T, static_cast<int>(K), static_cast<int>(cin), static_cast<int>(cin2),
-                                  static_cast<int>(cout), has_map ? 1 : 0, SPIRA_OUT_STORE, &tn.k, plan),
+                                  static_cast<int>(cout), static_cast<int>(has_map), SPIRA_OUT_STORE, &tn.k, plan),
            "conv_os_plan");
   return std::vector<int64_t>(plan, plan + 7);
 }
