@@ -457,10 +457,11 @@ int spira_hip_conv_ws_fused(int64_t num_sources, int64_t num_targets, const int3
                             int c_in, const void *weights, const void *prepared, int num_weights, int c_out,
                             int dtype, float *target_acc, hipStream_t stream);
 
-/* Fragment-major copy of weights [K, c_in, c_out] for spira_hip_conv_map,
+/* Fragment-major copy of fp16 weights [K, c_in, c_out] for spira_hip_conv_map,
  * conv_masks and conv_pairs: per offset, 16-column tile and 64 bytes of input
  * channels, one 1 KB block in the lane order of the matrix instructions,
- * zero-padded.  Valid until the weights change.  (No reference counterpart.) */
+ * zero-padded.  Valid until the weights change.  fp32 weights have none (0
+ * bytes): the kernels read them as they are.  (No reference counterpart.) */
 int spira_hip_fragments_bytes(int num_offsets, int c_in, int c_out, int dtype, size_t *bytes);
 int spira_hip_prepare_fragments(const void *weights, int num_offsets, int c_in, int c_out, int dtype, void *fragments,
                                 hipStream_t stream);

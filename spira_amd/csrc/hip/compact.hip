@@ -57,10 +57,11 @@ struct Entries {
 struct Layer {
   const void *X;  // [S, Cin], rows of a multiple of 16 bytes
   uint32_t xbytes, rowbytes;
-  const void *F;  // fragment-major weights (spira_hip_prepare_fragments)
+  const void *F;  // fp16: fragment-major weights (spira_hip_prepare_fragments)
   int ctiles, nft;  // 16-column tiles, and 64-byte fragments per input row
   int Cout;
-  const void *W;  // [K, Cin, Cout] (repeated pairs only)
+  const void *W;  // [K, Cin, Cout] (fp32, and repeated pairs)
+  uint32_t wbytes;  // of one offset
   int Cin;
   void *Y;         // [T, Cout]
   const float *scale, *shift;
@@ -139,7 +140,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC))) 
   constexpr int UT = U / 16;                       // tiles per unit
   constexpr int LPR = PITCH / 16, RPI = 64 / LPR;  // lanes per row, rows per DMA
   constexpr int IA = (U / RPI + NW - 1) / NW;      // DMAs per wave and step
-  constexpr int LPS = IA + NF * NC;                // vector-memory loads per wave and step
+  constexpr int LPS = IA + NF * NC * (sizeof(FT) == 4 ? 4 : 1);  // vector-memory loads per wave and step
   constexpr int STAGE = IA * NW * 1024;
   constexpr int MAXU = CH * ((BT + U - 1) / U);
   static_assert(BT % 64 == 0 && BT <= 128 && CH <= 32 && NT % CH == 0, "chunk shape");
@@ -348,7 +349,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC))) 
       const uint32_t tb = tgt_at + kl * BT + ((nd >> 8) & 255) + l16;
       unroll<UT>([&](auto I) { tg[s][decltype(I)::value] = rd1<decltype(I)::value * 16>(tb); });
       const int f0 = ich * NF;
-      const floatx4 *wp = static_cast<const floatx4 *>(l.F) + (static_cast<int64_t>(c0 + kl) * l.ctiles * l.nft + f0) * 64 + lane;
       if (++ich == nch) {
         ich = 0;
         iunit = iunit + 1 < nunits ? iunit + 1 : iunit;
@@ -366,10 +366,32 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC))) 
 #pragma unroll
       for (int j = 0; j < UT; ++j) pin(tg[s][j]);
       peek(un);
+      if constexpr (sizeof(FT) == 4) {
+        // fp32 weights as they are, so that no copy of them can be stale: the
+        // lane's four channels of its column (a quarter wave on 64 bytes of a
+        // row; past Cin out of the offset's range, zero; past Cout the next
+        // row's values, in columns that are not stored).  20k voxels, 32 -> 32
+        // 29.3 us, from fragments kept from call to call 27.9.
+        const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<char *>(static_cast<const char *>(l.W) + static_cast<int64_t>(c0 + kl) * l.wbytes), 0,
+            static_cast<int>(l.wbytes), 0x00020000);
 #pragma unroll
-      for (int q = 0; q < NC; ++q)
+        for (int q = 0; q < NC; ++q)
 #pragma unroll
-        for (int f = 0; f < NF; ++f) wf[s][f][q] = wp[(ct[q] * l.nft + f) * 64];
+          for (int f = 0; f < NF; ++f)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              wf[s][f][q][e] = __builtin_bit_cast(
+                  float, __builtin_amdgcn_raw_buffer_load_b32(
+                             wr, (((f0 + f) * 16 + lq * 4 + e) * l.Cout + ct[q] * 16 + l16) * 4, 0, 0));
+      } else {
+        const floatx4 *wp = static_cast<const floatx4 *>(l.F) +
+                            (static_cast<int64_t>(c0 + kl) * l.ctiles * l.nft + f0) * 64 + lane;
+#pragma unroll
+        for (int q = 0; q < NC; ++q)
+#pragma unroll
+          for (int f = 0; f < NF; ++f) wf[s][f][q] = wp[(ct[q] * l.nft + f) * 64];
+      }
       peeked();
     };
     // the products of J + 1 tiles of stage i
@@ -519,22 +541,20 @@ __global__ __launch_bounds__(256) void pair_rows_kernel(const int32_t *__restric
   if (Kw > 0 && 2 * lo + 1 != Kw) put(Kw - 1 - lo, b, a);
 }
 
-// fragment-major weights: 1 KB blocks (offset k, 16-column tile c, fragment f),
-// lane l's 16 bytes = input channels of quarter l / 16 of the fragment, output
-// column 16 c + l % 16; zero past Cin and Cout
-template <class FT>
-__global__ __launch_bounds__(256) void fragments_kernel(const FT *__restrict__ W, int64_t n, int Cin, int Cout,
-                                                        int ctiles, int nft, FT *__restrict__ F) {
-  constexpr int V = 16 / sizeof(FT);
+// fragment-major fp16 weights: 1 KB blocks (offset k, 16-column tile c,
+// fragment f), lane l's 16 bytes = input channels of quarter l / 16 of the
+// fragment, output column 16 c + l % 16; zero past Cin and Cout
+__global__ __launch_bounds__(256) void fragments_kernel(const _Float16 *__restrict__ W, int64_t n, int Cin, int Cout,
+                                                        int ctiles, int nft, _Float16 *__restrict__ F) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;  // one lane's 16 bytes
   if (i >= n) return;
   const int lane = static_cast<int>(i & 63);
   const int64_t blk = i >> 6, k = blk / (static_cast<int64_t>(ctiles) * nft);
   const int rem = static_cast<int>(blk % (static_cast<int64_t>(ctiles) * nft));
-  const int co = rem / nft * 16 + (lane & 15), ci = (rem % nft * 4 + (lane >> 4)) * V;
+  const int co = rem / nft * 16 + (lane & 15), ci = (rem % nft * 4 + (lane >> 4)) * 8;
 #pragma unroll
-  for (int e = 0; e < V; ++e)
-    F[i * V + e] = (co < Cout && ci + e < Cin) ? W[(k * Cin + ci + e) * Cout + co] : static_cast<FT>(0.f);
+  for (int e = 0; e < 8; ++e)
+    F[i * 8 + e] = (co < Cout && ci + e < Cin) ? W[(k * Cin + ci + e) * Cout + co] : static_cast<_Float16>(0.f);
 }
 
 // Rows padded with zero channels to 16 bytes
@@ -621,8 +641,8 @@ int spira_hip_conv_compact_workspace(int64_t num_sources, int64_t num_targets, i
 }  // extern "C"
 
 static size_t fragments_bytes(int num_offsets, int c_in, int c_out, int dtype) {
-  const int v = dtype == SPIRA_F16 ? 8 : 4;
-  return static_cast<size_t>(num_offsets) * div_up(c_out, 16) * div_up(c_in, 4 * v) * 1024;
+  if (dtype != SPIRA_F16) return 0;
+  return static_cast<size_t>(num_offsets) * div_up(c_out, 16) * div_up(c_in, 32) * 1024;
 }
 
 static int check_compact(int64_t num_sources, int64_t num_targets, int row_channels, int c_in, int c_out, int dtype,
@@ -636,8 +656,10 @@ static int check_compact(int64_t num_sources, int64_t num_targets, int row_chann
   SPIRA_HIP_REQUIRE(num_sources >= 0 && num_sources * row_channels * (16 / v) < (int64_t(1) << 31) &&
                         num_targets < (int64_t(1) << 31) - 256,
                     "conv_compact: features of one layer must stay below 2 GiB");
-  SPIRA_HIP_REQUIRE(fragments != nullptr && weights != nullptr,
-                    "conv_compact: needs the weights and their fragments (spira_hip_prepare_fragments)");
+  SPIRA_HIP_REQUIRE(weights != nullptr && (fragments != nullptr || dtype == SPIRA_F32),
+                    "conv_compact: needs the weights and, in fp16, their fragments (spira_hip_prepare_fragments)");
+  SPIRA_HIP_REQUIRE((static_cast<int64_t>(c_in) + 64) * c_out * 4 < (int64_t(1) << 31),
+                    "conv_compact: weights of one offset must stay below 2 GiB");
   return kOk;
 }
 
@@ -654,6 +676,7 @@ static compact::Layer make_layer(const void *sources, int64_t num_sources, int r
   l.nft = static_cast<int>(div_up(c_in * size, 64));
   l.Cout = c_out;
   l.W = weights;
+  l.wbytes = static_cast<uint32_t>(static_cast<int64_t>(c_in) * c_out * size);
   l.Cin = c_in;
   l.Y = targets;
   l.scale = scale;
@@ -677,16 +700,10 @@ int spira_hip_prepare_fragments(const void *weights, int num_offsets, int c_in, 
   SPIRA_HIP_REQUIRE(dtype == SPIRA_F16 || dtype == SPIRA_F32, "prepare_fragments: dtype must be fp16 or fp32");
   const int64_t n = static_cast<int64_t>(fragments_bytes(num_offsets, c_in, c_out, dtype) / 16);
   if (n == 0) return kOk;
-  const int ctiles = static_cast<int>(div_up(c_out, 16)), v = dtype == SPIRA_F16 ? 8 : 4;
-  const int nft = static_cast<int>(div_up(c_in, 4 * v));
-  if (dtype == SPIRA_F16)
-    hipLaunchKernelGGL(compact::fragments_kernel<_Float16>, dim3(div_up(n, 256)), dim3(256), 0, stream,
-                       static_cast<const _Float16 *>(weights), n, c_in, c_out, ctiles, nft,
-                       static_cast<_Float16 *>(fragments));
-  else
-    hipLaunchKernelGGL(compact::fragments_kernel<float>, dim3(div_up(n, 256)), dim3(256), 0, stream,
-                       static_cast<const float *>(weights), n, c_in, c_out, ctiles, nft,
-                       static_cast<float *>(fragments));
+  const int ctiles = static_cast<int>(div_up(c_out, 16)), nft = static_cast<int>(div_up(c_in, 32));
+  hipLaunchKernelGGL(compact::fragments_kernel, dim3(div_up(n, 256)), dim3(256), 0, stream,
+                     static_cast<const _Float16 *>(weights), n, c_in, c_out, ctiles, nft,
+                     static_cast<_Float16 *>(fragments));
   SPIRA_HIP_LAUNCH_CHECK();
   return kOk;
 }

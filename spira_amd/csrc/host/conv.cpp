@@ -88,13 +88,17 @@ static torch::Tensor prepared_weights(const torch::Tensor &W) {
   return cached_copy(cache, W, bytes, &spira_hip_prepare_weights);
 }
 
-// Returns the fragment-major copy of W (the compacted kernels' weights).
+// Returns the fragment-major copy of fp16 W (the compacted kernels' weights;
+// fp32 weights are read as they are, as by every fp32 kernel, so that they may
+// change in any way between two calls: undefined).
 static torch::Tensor weight_fragments(const torch::Tensor &W) {
   static PreparedCache cache;
   size_t bytes = 0;
   check_rc(spira_hip_fragments_bytes(W.size(0), W.size(1), W.size(2), dtype_of(W), &bytes), "prepare_fragments");
+  if (bytes == 0) return torch::Tensor();
   return cached_copy(cache, W, bytes, &spira_hip_prepare_fragments);
 }
+static const void *ptr_or_null(const torch::Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
 
 // Source rows as the compacted kernels gather them: padded with zero channels
 // to 16-byte rows, on a 16-byte boundary.
@@ -110,10 +114,12 @@ static torch::Tensor compact_rows(const torch::Tensor &X) {
   return reinterpret_cast<uintptr_t>(X.data_ptr()) % 16 == 0 ? X : X.clone();
 }
 
-// The compacted kernels address the source rows with 31-bit byte offsets.
-static bool compact_fits(const torch::Tensor &X) {
+// The compacted kernels address the source rows and an offset's weights with
+// 31-bit byte offsets.
+static bool compact_fits(const torch::Tensor &X, const torch::Tensor &W) {
   const int64_t v = 16 / X.element_size();
-  return X.size(0) * ((X.size(1) + v - 1) / v * 16) < (int64_t(1) << 31);
+  return X.size(0) * ((X.size(1) + v - 1) / v * 16) < (int64_t(1) << 31) &&
+         (W.size(1) + 64) * W.size(2) * 4 < (int64_t(1) << 31);
 }
 
 // pointer to weight row `k` of W, and of its prepared copy
@@ -503,11 +509,10 @@ static void run_os(const torch::Tensor *map, int64_t S, int64_t T, const torch::
   // pad first (a launch of its own: 3 -> 32 channels down-sampling 5k voxels
   // 12 -> 16 us; 20k targets x 8 offsets and more are faster with it)
   const bool small_unaligned = X.size(1) % 4 != 0 && T * K < 200000;
-  if (dtype == SPIRA_F32 && mp && mode == SPIRA_OUT_STORE && T > 0 && !small_unaligned && compact_fits(X)) {
-    auto F = weight_fragments(W);
+  if (dtype == SPIRA_F32 && mp && mode == SPIRA_OUT_STORE && T > 0 && !small_unaligned && compact_fits(X, W)) {
     auto Xr = compact_rows(X);
     check_rc(spira_hip_conv_map(X.size(0), T, K, mp, Xr.data_ptr(), Xr.size(1), W.size(1), wrow_ptr(W, w0),
-                                F.data_ptr(), W.size(2), dtype, out, epi.scale, epi.shift, epi.residual, epi.relu,
+                                nullptr, W.size(2), dtype, out, epi.scale, epi.shift, epi.residual, epi.relu,
                                 current_stream()),
              "sparse_convolution_forward_os");
     return;
@@ -673,7 +678,7 @@ static bool masks_compact(int64_t S, int64_t T, const torch::Tensor &X, const to
                           const torch::Tensor &source_masks, const torch::Tensor &target_masks,
                           const torch::Tensor &nbsizes, bool half, const torch::Tensor *dense, int Kos, const Epi &e,
                           torch::Tensor &Y) {
-  if (!compact_fits(X) || W.numel() == 0) return false;
+  if (!compact_fits(X, W) || W.numel() == 0) return false;
   check_masks(S, T, source_masks, target_masks);
   const int Km = static_cast<int>(target_masks.size(0));
   const int nh = half ? (Km + 1) / 2 : Km;
@@ -686,7 +691,7 @@ static bool masks_compact(int64_t S, int64_t T, const torch::Tensor &X, const to
   auto ws = workspace(wsb, X.device());
   check_rc(spira_hip_conv_masks(S, T, Km, source_masks.data_ptr<int32_t>(), target_masks.data_ptr<int32_t>(), Kos,
                                 dense ? dense->data_ptr<int32_t>() : nullptr, Xr.data_ptr(), Xr.size(1), W.size(1),
-                                W.data_ptr(), F.data_ptr(), W.size(2), dtype_of(X), Y.data_ptr(), e.scale, e.shift,
+                                W.data_ptr(), ptr_or_null(F), W.size(2), dtype_of(X), Y.data_ptr(), e.scale, e.shift,
                                 e.residual, e.relu, ws.data_ptr(), wsb, current_stream()),
            "gather");
   return true;
@@ -800,7 +805,7 @@ static std::optional<torch::Tensor> pairs_compact(int64_t S, int64_t T, const to
                           int64_t mapsize, bool transpose, int mirror_rows, const torch::Tensor *dense, int Kos,
                           const Epi &e) {
   const int rows = static_cast<int>(naddrs.size(0) - 1);
-  if (!compact_fits(X) || W.numel() == 0 || mapsize >= (int64_t(1) << 29)) return std::nullopt;
+  if (!compact_fits(X, W) || W.numel() == 0 || mapsize >= (int64_t(1) << 29)) return std::nullopt;
   // (about T pairs in a self-mirrored centre row, taken once, and in a
   // hybrid's dense offsets)
   const int64_t pairs = (mirror_rows > 0 ? 2 : 1) * mapsize - (mirror_rows % 2 == 1 ? T : 0) + (Kos > 0 ? T : 0);
@@ -818,7 +823,7 @@ static std::optional<torch::Tensor> pairs_compact(int64_t S, int64_t T, const to
   auto ws = workspace(wsb, X.device());
   check_rc(spira_hip_conv_pairs(S, T, imap, omap, rows, naddrs.data_ptr<int32_t>(), mapsize, mirror_rows, Kos,
                                 dense ? dense->data_ptr<int32_t>() : nullptr, Xr.data_ptr(), Xr.size(1), W.size(1),
-                                W.data_ptr(), F.data_ptr(), W.size(2), dtype_of(X), Y.data_ptr(), e.scale, e.shift,
+                                W.data_ptr(), ptr_or_null(F), W.size(2), dtype_of(X), Y.data_ptr(), e.scale, e.shift,
                                 e.residual, e.relu, ws.data_ptr(), wsb, current_stream()),
            "sparse_convolution_forward_ws_merged");
   return Y;
