@@ -217,9 +217,12 @@ class SparseConv(Module):
     def reset_parameters(self) -> None:
         fan = self.out_channels if self.transposed else self.in_channels
         bound = 1.0 / np.sqrt(fan * len(self.kernel))
-        self.kernel.data.uniform_(-bound, bound)
-        if self.bias is not None:
-            self.bias.data.uniform_(-bound, bound)
+        # (through the parameter itself: a write to its .data leaves its version,
+        # by which fp16 layers know that their prepared weights are stale)
+        with torch.no_grad():
+            self.kernel.uniform_(-bound, bound)
+            if self.bias is not None:
+                self.bias.uniform_(-bound, bound)
 
     def set_kernel_map_cache(self, cache: KernelMapCache) -> None:
         self._kernel_map_cache = cache

@@ -19,6 +19,15 @@ from helpers import np_, rel_err
 DATAFLOWS = [0, 1, 2, 3, 5, 6]
 
 
+def test_reset_parameters_is_seen():
+    """A reset counts as a change of the parameters (their version)."""
+    m = spnn.SparseConv(4, 8, 3, bias=True)
+    before = m.kernel._version, m.bias._version
+    m.reset_parameters()
+    assert m.kernel._version > before[0] and m.bias._version > before[1]
+    assert m.kernel.requires_grad
+
+
 @pytest.fixture(scope="module")
 def keys(dev):
     k, _ = orc.flatten_sort(1 + scenes.spheres_planes(n=6000, grid=64, seed=3), True)
@@ -65,6 +74,19 @@ def test_float32_weights_changed_in_place(dev, keys, d):
         conv.kernel.add_(1.0)
         seen.append(check())
     assert all(not torch.equal(a, b) for a, b in zip(seen, seen[1:]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [0, 1, 2])
+def test_float16_reset_parameters(dev, keys, d):
+    conv, x = _layer(keys, d, dtype=torch.float16)
+    fresh, _ = _layer(keys, d, dtype=torch.float16)
+    with torch.no_grad():
+        for _ in range(2):
+            y = conv(x).features
+            fresh.kernel = torch.nn.Parameter(conv.kernel.detach().clone())
+            assert rel_err(np_(y.float()), np_(fresh(x).features.float())) <= 4e-3
+            conv.reset_parameters()
 
 
 @pytest.mark.gpu
