@@ -766,7 +766,8 @@ int spira_hip_conv_masks(int64_t num_sources, int64_t num_targets, int num_offse
     SPIRA_HIP_LAUNCH_CHECK();
   }
   compact::Entries en{};
-  en.kind = compact::kMasks;
+  // (without masked offsets there are no ranks to look up, and no list)
+  en.kind = num_offsets > 0 ? compact::kMasks : compact::kRowsKT;
   en.idx = target_masks;
   en.ld = num_targets;
   en.list = list;

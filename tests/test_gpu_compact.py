@@ -6,6 +6,9 @@ pairs in any order and repeated pairs.  Against a float64 sum over the pairs.
 Tolerance, max |error| / RMS(reference): fp16 stores round to 2^-11 of a value
 that may be 6 x RMS (3e-3) -> 4e-3; fp32 sums of up to 8000 products, error
 growth ~ sqrt(n) 2^-24 of the terms' norm -> 1e-5 (the fp32 bar)."""
+import ctypes
+import os
+
 import numpy as np
 import pytest
 import torch
@@ -133,3 +136,37 @@ def test_values_stay_in_their_rows(dev):
         touched[t[(s == 7) | (s == 90)]] = True
     assert not np.isfinite(y[touched]).any(axis=1).any() or np.isnan(y[touched]).any(axis=1).all()
     assert np.isfinite(y[~touched]).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("Kd", [1, 2, 8])
+def test_hybrid_without_masked_offsets(dev, dtype, Kd):
+    """A hybrid of dense offsets alone (Kd 1: the identity), through the C entry
+    with the null workspace that its query allows and through the torch layer."""
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "spira_amd",
+                                   "libspira_hip.so"))
+    S = T = 130
+    g = torch.Generator().manual_seed(Kd)
+    m = torch.randint(-S, S, (T, Kd), generator=g, dtype=torch.int32).clamp_(min=-1)
+    if Kd == 1:
+        m = torch.arange(T, dtype=torch.int32)[:, None]
+    X, W, _ = _data(S, T, Kd, 32, 48, dtype, Kd)
+    lists = [(m[m[:, k] >= 0, k].numpy(), torch.nonzero(m[:, k] >= 0)[:, 0].numpy()) for k in range(Kd)]
+    Xd, Wd = X.to(dev), W.to(dev)
+    dense = None if Kd == 1 else torch.nn.functional.pad(m, (0, 0, 0, -T % 128), value=-1).to(dev)
+    none = torch.empty(0, S, dtype=torch.int32, device=dev)
+    y = F.sparse_convolution_forward_hs(S, T, Xd, Wd, none, none, torch.empty(0, dtype=torch.int32, device=dev), dense,
+                                        16, 16)
+    assert rel_err(np_(y.float()), _ref(lists, T, X, W)) <= TOL[dtype]
+    size = ctypes.c_size_t()
+    code = 0 if dtype == torch.float16 else 1
+    assert lib.spira_hip_fragments_bytes(Kd, 32, 48, code, ctypes.byref(size)) == 0
+    frag = torch.empty(max(size.value, 1), dtype=torch.uint8, device=dev)
+    out = torch.empty(T, 48, dtype=dtype, device=dev)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ptr = lambda t: ctypes.c_void_p(None if t is None else t.data_ptr())
+    assert lib.spira_hip_prepare_fragments(ptr(Wd), Kd, 32, 48, code, ptr(frag), stream) == 0
+    assert lib.spira_hip_conv_masks(ctypes.c_int64(S), ctypes.c_int64(T), 0, None, None, Kd, ptr(dense), ptr(Xd), 32,
+                                    32, ptr(Wd), ptr(frag), 48, code, ptr(out), None, None, None, 0, None,
+                                    ctypes.c_size_t(0), stream) == 0
+    assert rel_err(np_(out.float()), _ref(lists, T, X, W)) <= TOL[dtype]
