@@ -5,11 +5,13 @@
 // torch/cuda_memory_buffer.cu:7-16.
 #include "host_common.h"
 
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/hip/HIPCachingAllocator.h>
 
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <memory>
 #include <tuple>
 #include <unordered_map>
 
@@ -28,17 +30,19 @@ static int dtype_of(const torch::Tensor &t) {
 // while that kernel still reads it (an order overwritten under a running
 // convolution indexes its output rows out of bounds).
 static void record_use(hipStream_t made_on, std::initializer_list<const torch::Tensor *> ts) {
-  const auto cur = c10::hip::getCurrentHIPStream();
+  // (in the form that tensors of a "cuda" device take)
+  const auto cur = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA();
   if (cur.stream() == made_on) return;
   for (const torch::Tensor *t : ts)
-    if (t->defined()) const_cast<torch::Tensor *>(t)->record_stream(cur);
+    if (t->defined()) const_cast<torch::Tensor *>(t)->record_stream(cur.unwrap());
 }
 
 // Prepared (MFMA-ready) weights, cached per weight tensor.  An entry is valid
 // while the same TensorImpl is alive with the same storage pointer and
 // version counter, so an optimizer step or `param.data = ...` invalidates it;
 // the weak reference keeps a freed tensor's address from being reused by a
-// different tensor while its entry exists.
+// different tensor while its entry exists.  Other streams wait for `written`
+// before they read the copy.
 struct PreparedEntry {
   explicit PreparedEntry(const torch::Tensor &w) : impl(w.getIntrusivePtr()) {}
   c10::weak_intrusive_ptr<c10::TensorImpl> impl;
@@ -46,12 +50,21 @@ struct PreparedEntry {
   uint32_t version = 0;
   torch::Tensor prepared;
   hipStream_t stream = nullptr;  // the stream that allocated and wrote `prepared`
+  std::shared_ptr<ihipEvent_t> written;
 };
+
+static bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
 
 using PreparedCache = std::unordered_map<const c10::TensorImpl *, PreparedEntry>;
 using PrepareFn = int (*)(const void *, int, int, int, int, void *, hipStream_t);
 
-// The copy of W that `prepare` writes, from `cache` or made now.
+// The copy of W that `prepare` writes, from `cache` or made now.  A copy made
+// while the stream is captured is written by the graph's replays alone and is
+// not kept; a kept one is taken under capture as it is (whoever begins a
+// capture has synchronized the device).
 static torch::Tensor cached_copy(PreparedCache &cache, const torch::Tensor &W, size_t bytes, PrepareFn prepare) {
   const int dtype = dtype_of(W);
   const c10::TensorImpl *key = W.unsafeGetTensorImpl();
@@ -60,10 +73,19 @@ static torch::Tensor cached_copy(PreparedCache &cache, const torch::Tensor &W, s
     auto &e = it->second;
     if (!e.impl.expired() && e.data == W.data_ptr() && e.version == W._version() &&
         e.prepared.device() == W.device()) {
+      const hipStream_t s = current_stream();
+      if (s != e.stream && !capturing(s))
+        SPIRA_CHECK_ARG(hipStreamWaitEvent(s, e.written.get(), 0) == hipSuccess, "stream wait failed");
       record_use(e.stream, {&e.prepared});
       return e.prepared;
     }
     cache.erase(it);
+  }
+  if (capturing(current_stream())) {
+    auto copy = workspace(bytes, W.device());
+    check_rc(prepare(W.data_ptr(), W.size(0), W.size(1), W.size(2), dtype, copy.data_ptr(), current_stream()),
+             "prepare_weights");
+    return copy;
   }
   // drop the entries of freed weight tensors (one entry per live layer)
   for (auto i = cache.begin(); i != cache.end();) i = i->second.impl.expired() ? cache.erase(i) : std::next(i);
@@ -74,6 +96,10 @@ static torch::Tensor cached_copy(PreparedCache &cache, const torch::Tensor &W, s
   e.stream = current_stream();
   check_rc(prepare(W.data_ptr(), W.size(0), W.size(1), W.size(2), dtype, e.prepared.data_ptr(), current_stream()),
            "prepare_weights");
+  hipEvent_t written = nullptr;
+  SPIRA_CHECK_ARG(hipEventCreateWithFlags(&written, hipEventDisableTiming) == hipSuccess, "event creation failed");
+  e.written.reset(written, [](hipEvent_t ev) { (void)hipEventDestroy(ev); });
+  SPIRA_CHECK_ARG(hipEventRecord(written, e.stream) == hipSuccess, "event record failed");
   auto out = e.prepared;
   cache.emplace(key, std::move(e));
   return out;

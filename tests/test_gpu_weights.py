@@ -142,3 +142,51 @@ def test_float32_captured(dev, keys, d):
             assert torch.equal(got, conv(x).features)
             conv.kernel.data.mul_(1.0 + i)
             torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", DATAFLOWS)
+def test_float16_prepared_for_another_stream(dev, keys, d):
+    """Weights prepared on a busy stream are waited for by the stream that
+    reads them next."""
+    conv, x = _layer(keys, d, dtype=torch.float16)
+    twin, _ = _layer(keys, d, dtype=torch.float16)
+    twin.set_kernel_map_cache(conv._kernel_map_cache)
+    twin.kernel = torch.nn.Parameter(conv.kernel.detach().clone())
+    with torch.no_grad():
+        want = twin(x).features  # (the map is made here)
+        torch.cuda.synchronize()
+        a, b = torch.cuda.Stream(), torch.cuda.Stream()
+        with torch.cuda.stream(a):
+            torch.cuda._sleep(20_000_000)  # ~10 ms
+            ya = conv(x).features
+        with torch.cuda.stream(b):
+            yb = conv(x).features
+        torch.cuda.synchronize()
+    for y in (ya, yb):
+        assert rel_err(np_(y.float()), np_(want.float())) <= 4e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [0, 1, 2, 6])
+def test_float16_captured_first(dev, keys, d):
+    """A layer whose first call is captured: eager calls before a replay and
+    after it, and every replay, compute the same."""
+    conv, x = _layer(keys, d, dtype=torch.float16)
+    twin, _ = _layer(keys, d, dtype=torch.float16)
+    for m in (conv, twin):  # (one part: no workspace shared by the stream's calls)
+        m.tunable_config["os_tuning"] = (0, 0, 1, 0, 0, 0)
+    twin.set_kernel_map_cache(conv._kernel_map_cache)
+    twin.kernel = torch.nn.Parameter(conv.kernel.detach().clone())
+    with torch.no_grad():
+        want = np_(twin(x).features.float())
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = conv(x).features
+        for _ in range(3):
+            assert rel_err(np_(conv(x).features.float()), want) <= 4e-3
+            y.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert rel_err(np_(y.float()), want) <= 4e-3
