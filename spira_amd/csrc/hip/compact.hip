@@ -515,14 +515,16 @@ __global__ __launch_bounds__(256) void rows_clear_kernel(int32_t *__restrict__ r
 }
 
 // rows[k, out] = in for the pairs of compacted row k, and with Kw > 0 the
-// mirrored rows[Kw - 1 - k, in] = out (a self-mirrored centre row once)
+// mirrored rows[Kw - 1 - k, in] = out (a self-mirrored centre row once); pairs
+// past the last row's, or with an index outside its side (-1), are none
 __global__ __launch_bounds__(256) void pair_rows_kernel(const int32_t *__restrict__ in_idx,
                                                         const int32_t *__restrict__ out_idx,
                                                         const int32_t *__restrict__ naddrs, int R, int64_t P, int Kw,
-                                                        int64_t ld, int32_t *__restrict__ rows,
+                                                        int64_t S, int64_t T, int64_t ld,
+                                                        int32_t *__restrict__ rows,
                                                         int32_t *__restrict__ extra, int32_t *__restrict__ nextra) {
   const int64_t p = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (p >= P) return;
+  if (p >= P || p >= naddrs[R]) return;
   int lo = 0, hi = R;  // last row with naddrs[row] <= p
   while (hi - lo > 1) {
     const int m = (lo + hi) >> 1;
@@ -537,8 +539,9 @@ __global__ __launch_bounds__(256) void pair_rows_kernel(const int32_t *__restric
     extra[3 * at + 2] = t;
   };
   const int32_t a = in_idx[p], b = out_idx[p];
+  if (a < 0 || a >= S || b < 0 || b >= T) return;
   put(lo, a, b);
-  if (Kw > 0 && 2 * lo + 1 != Kw) put(Kw - 1 - lo, b, a);
+  if (Kw > 0 && 2 * lo + 1 != Kw && b < S && a < T) put(Kw - 1 - lo, b, a);
 }
 
 // fragment-major fp16 weights: 1 KB blocks (offset k, 16-column tile c,
@@ -802,7 +805,8 @@ int spira_hip_conv_pairs(int64_t num_sources, int64_t num_targets, const int32_t
   SPIRA_HIP_LAUNCH_CHECK();
   if (num_pairs > 0) {
     hipLaunchKernelGGL(compact::pair_rows_kernel, dim3(div_up(num_pairs, 256)), dim3(256), 0, stream, in_idx, out_idx,
-                       naddrs, rows, num_pairs, mirror_rows, ld, idx, extra, nextra);
+                       naddrs, rows, num_pairs, mirror_rows, num_sources, num_targets, ld, idx, extra,
+                       nextra);
     SPIRA_HIP_LAUNCH_CHECK();
   }
   compact::Entries en{};

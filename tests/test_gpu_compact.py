@@ -89,6 +89,20 @@ def test_fp32_map(dev, S, T, K, cin, cout, density):
     assert rel_err(np_(y), _ref(lists, T, X, W, epi)) <= TOL[torch.float32]
 
 
+def _pair_list(lists, dev, unused=0):
+    """(naddrs, qnaddrs, nbmaps) on the device; with `unused` every 40th entry
+    -1 on one side and that many entries past the last row's."""
+    sizes = np.array([len(s) for s, _ in lists])
+    naddrs = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    qn = np.concatenate([[0], np.cumsum((sizes + 127) // 128 * 128)]).astype(np.int32)
+    nb = np.stack([np.concatenate([s for s, _ in lists]), np.concatenate([t for _, t in lists])]).astype(np.int32)
+    if unused:
+        nb[0, 7::80] = -1
+        nb[1, 47::80] = -1
+        nb = np.concatenate([nb, np.zeros((2, unused), np.int32)], 1)
+    return [torch.from_numpy(np.ascontiguousarray(a)).to(dev) for a in (naddrs, qn, nb)]
+
+
 @pytest.mark.parametrize("repeat", [False, True])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("S,T,K,cin,cout", [(2100, 2000, 27, 64, 64), (1500, 1400, 8, 96, 100), (900, 901, 40, 128, 48)])
@@ -113,6 +127,47 @@ def test_pairs(dev, dtype, S, T, K, cin, cout, repeat):
     y = F.sparse_convolution_forward_ws_merged(T, S, X2.to(dev), W.to(dev), d(naddrs), d(qn), d(nb), nb.shape[1],
                                                int(qn[-1]), True)
     assert rel_err(np_(y.float()), _ref(back, S, X2, W)) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("unused", [0, 100])
+@pytest.mark.parametrize("repeat", [0, 7])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("dense", [-1, 0, 3])
+def test_mirrored_pairs(dev, dtype, dense, repeat, unused):
+    """Half a submanifold layer's pairs, each counted for its mirrored offset
+    too: alone (dense -1; the centre row once), or as a hybrid beside an identity
+    or a map of dense offsets.  Repeated pairs count twice, entries of -1 and
+    past the last row's not at all."""
+    S = T = 2501
+    K, cin, cout = 27, 64, 64
+    rows = 14 if dense < 0 else 12
+    rng = np.random.default_rng(dense + 5)
+    lists = _lists(S, T, rows, 0.6, 11)
+    if repeat:
+        lists = [(np.concatenate([s, s[::repeat]]), np.concatenate([t, t[::repeat]])) for s, t in lists]
+    naddrs, qn, nb = _pair_list(lists, dev, unused)
+    ends = np_(naddrs)
+    kept = []
+    for r in range(rows):
+        s, t = np_(nb)[:, ends[r]:ends[r + 1]]
+        ok = (s >= 0) & (t >= 0)
+        kept.append((s[ok], t[ok]))
+    Kos = {-1: 0, 0: 1, 3: 3}[dense]
+    Kw = 27 if dense < 0 else 2 * rows
+    full = kept + [(t, s) for s, t in kept[::-1]][Kw % 2:]
+    X, W, epi = _data(S, T, Kw + Kos, cin, cout, dtype, 1)
+    args = (X.to(dev), W.to(dev), naddrs, qn, nb)
+    if dense < 0:
+        y = F.sparse_convolution_forward_ws_merged(S, T, *args, nb.shape[1], int(qn[-1]), epilogue=_dev(epi, dev))
+    else:
+        m, first = None, [(np.arange(T), np.arange(T))]
+        if dense:
+            m = np.maximum(rng.integers(-S, S, (T, Kos)), -1).astype(np.int32)
+            first = [(m[m[:, k] >= 0, k], np.nonzero(m[:, k] >= 0)[0]) for k in range(Kos)]
+            m = torch.from_numpy(m).to(dev)
+        y = F.sparse_convolution_forward_hs_merged(S, T, *args, m, nb.shape[1], int(qn[-1]), epilogue=_dev(epi, dev))
+        full = first + full
+    assert rel_err(np_(y.float()), _ref(full, T, X, W, epi)) <= TOL[dtype]
 
 
 def test_values_stay_in_their_rows(dev):
