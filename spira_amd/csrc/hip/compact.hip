@@ -49,10 +49,12 @@ struct Entries {
   const int32_t *dense;
   int kd;
   // pairs that lost their place in idx to another pair of the same target and
-  // offset: extra[0 .. *nextra), (offset, source, target) each; or null
-  const int32_t *extra;
-  const int32_t *nextra;
+  // offset: (offset, source, target, next of the block or -1) each, the first
+  // of block b at heads[b]; or null
+  const int4 *extra;
+  const int32_t *heads;
 };
+constexpr int kTargets = 64;  // targets per block
 
 struct Layer {
   const void *X;  // [S, Cin], rows of a multiple of 16 bytes
@@ -143,7 +145,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC))) 
   constexpr int LPS = IA + NF * NC * (sizeof(FT) == 4 ? 4 : 1);  // vector-memory loads per wave and step
   constexpr int STAGE = IA * NW * 1024;
   constexpr int MAXU = CH * ((BT + U - 1) / U);
-  static_assert(BT % 64 == 0 && BT <= 128 && CH <= 32 && NT % CH == 0, "chunk shape");
+  static_assert(BT == kTargets && BT % 64 == 0 && BT <= 128 && CH <= 32 && NT % CH == 0, "chunk shape");
   static_assert(PITCH >= NF * 64 && (D - 2) * LPS < 64 && U <= BT && U % 16 == 0, "step shape");
   // Sums: row t holds the 16-column chunks of target t (row BT takes the
   // padding pairs' products); chunk w sits at w ^ swz(t), so that 16 rows'
@@ -444,24 +446,36 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC))) 
   }
   __syncthreads();
   const FT *X = static_cast<const FT *>(l.X);
-  if (en.nextra) {
+  if (en.heads) {
     // repeated (offset, target) pairs, none in a map's own lists: each one's
-    // product, a thread per column (in list order)
+    // product, four lanes per column (in any order).  Bound by the latency of
+    // its loads: 100k voxels, fp16 64 -> 64, every 1000th / 100th / 10th of a
+    // list's pairs repeated 66 / 71 / 123 us, none 48 (every block on one list,
+    // a lane per column: 244 / 520 / 4483; the fused pass 81 / 81 / 85).
     const FT *W = static_cast<const FT *>(l.W);
     const int64_t xs = l.rowbytes / sizeof(FT);
-    const int ne = *en.nextra;
-    for (int p = 0; p < ne; ++p) {
-      const int64_t k = en.extra[3 * p] + en.kd, s = en.extra[3 * p + 1];
-      const int64_t tl = en.extra[3 * p + 2] - t0;
-      if (tl < 0 || tl >= BT) continue;
-      for (int c = tid; c < BN && nb0 + c < l.Cout; c += NT) {
+    const int c0 = tid >> 2, q = tid & 3;
+    int p = en.heads[bx];
+    const bool any = p >= 0;
+    int4 e = any ? en.extra[p] : int4{};
+    while (p >= 0) {
+      const int64_t k = e.x + en.kd;
+      const FT *x = X + e.y * xs;
+      const int tl = static_cast<int>(e.z - t0);
+      p = e.w;
+      if (p >= 0) e = en.extra[p];
+      for (int c = c0; c < BN && nb0 + c < l.Cout; c += NT / 4) {  // (alike in the four lanes)
+        const FT *w = W + k * l.Cin * l.Cout + nb0 + c;
         float v = 0.f;
-        for (int ci = 0; ci < l.Cin; ++ci)
-          v = fmaf(static_cast<float>(X[s * xs + ci]), static_cast<float>(W[(k * l.Cin + ci) * l.Cout + nb0 + c]), v);
-        acc[at(static_cast<int>(tl), c / 16) + c % 16] += v;
+#pragma unroll 8
+        for (int ci = q; ci < l.Cin; ci += 4)
+          v = fmaf(static_cast<float>(x[ci]), static_cast<float>(w[static_cast<int64_t>(ci) * l.Cout]), v);
+        v += __shfl_xor(v, 1, 64);
+        v += __shfl_xor(v, 2, 64);
+        if (q == 0) acc[at(tl, c / 16) + c % 16] += v;
       }
     }
-    __syncthreads();
+    if (any) __syncthreads();
   }
   // output rows with the epilogue, 16 bytes per lane where rows are aligned
   constexpr int V = 16 / sizeof(FT);
@@ -516,13 +530,14 @@ __global__ __launch_bounds__(256) void rows_clear_kernel(int32_t *__restrict__ r
 
 // rows[k, out] = in for the pairs of compacted row k, and with Kw > 0 the
 // mirrored rows[Kw - 1 - k, in] = out (a self-mirrored centre row once); pairs
-// past the last row's, or with an index outside its side (-1), are none
+// past the last row's, or with an index outside its side (-1), are none.  A
+// repeated (offset, target) goes to the list of its block of targets.
 __global__ __launch_bounds__(256) void pair_rows_kernel(const int32_t *__restrict__ in_idx,
                                                         const int32_t *__restrict__ out_idx,
                                                         const int32_t *__restrict__ naddrs, int R, int64_t P, int Kw,
-                                                        int64_t S, int64_t T, int64_t ld,
-                                                        int32_t *__restrict__ rows,
-                                                        int32_t *__restrict__ extra, int32_t *__restrict__ nextra) {
+                                                        int64_t S, int64_t T, int64_t ld, int32_t *__restrict__ rows,
+                                                        int32_t *__restrict__ heads, int4 *__restrict__ extra,
+                                                        int32_t *__restrict__ nextra) {
   const int64_t p = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (p >= P || p >= naddrs[R]) return;
   int lo = 0, hi = R;  // last row with naddrs[row] <= p
@@ -534,9 +549,7 @@ __global__ __launch_bounds__(256) void pair_rows_kernel(const int32_t *__restric
   auto put = [&](int k, int32_t s, int32_t t) {
     if (atomicCAS(&rows[static_cast<int64_t>(k) * ld + t], -1, s) == -1) return;
     const int at = atomicAdd(nextra, 1);
-    extra[3 * at] = k;
-    extra[3 * at + 1] = s;
-    extra[3 * at + 2] = t;
+    extra[at] = make_int4(k, s, t, atomicExch(&heads[t / kTargets], at));
   };
   const int32_t a = in_idx[p], b = out_idx[p];
   if (a < 0 || a >= S || b < 0 || b >= T) return;
@@ -584,8 +597,8 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(const FT *__restrict__ X,
 template <class FT, int PITCH, int NF>
 static void launch_n(hipStream_t s, const Entries &en, int64_t T, int K, const Layer &l) {
 #define SPIRA_PAIR_CALL(NW, CH, D, OCC)                                                                         \
-  hipLaunchKernelGGL((pair_kernel<FT, PITCH, NF, NW, 1, 64, CH, 32, D, OCC>),                                   \
-                     dim3(static_cast<unsigned>(div_up(T, 64)), static_cast<unsigned>(div_up(l.ctiles, NW))), \
+  hipLaunchKernelGGL((pair_kernel<FT, PITCH, NF, NW, 1, kTargets, CH, 32, D, OCC>),                                   \
+                     dim3(static_cast<unsigned>(div_up(T, kTargets)), static_cast<unsigned>(div_up(l.ctiles, NW))), \
                      dim3(64 * NW), 0, s, en, T, K, l)
   constexpr int occ4 = PITCH == 256 ? 3 : 4;  // (what the ring leaves room for)
   if (l.Cout <= 16 && K <= 32) {
@@ -635,9 +648,11 @@ extern "C" {
 
 int spira_hip_conv_compact_workspace(int64_t num_sources, int64_t num_targets, int num_offsets, int64_t num_pairs,
                                      size_t *bytes) {
-  // masks: the sources by rank; pairs: entry rows by target, their overflow
+  // masks: the sources by rank; pairs: entry rows by target, the blocks' first
+  // repeated pair, their number and the repeated pairs
   const int64_t n = std::max(num_sources, round_up(num_targets, 4)) * std::max(num_offsets, 0);
-  *bytes = static_cast<size_t>(n + 4 + 6 * std::max<int64_t>(num_pairs, 0)) * sizeof(int32_t);
+  const int64_t heads = round_up(div_up(num_targets, compact::kTargets), 4);
+  *bytes = static_cast<size_t>(n + heads + 8 + 8 * std::max<int64_t>(num_pairs, 0)) * sizeof(int32_t);
   return kOk;
 }
 
@@ -796,17 +811,21 @@ int spira_hip_conv_pairs(int64_t num_sources, int64_t num_targets, const int32_t
   if (num_targets <= 0) return kOk;
   SPIRA_HIP_REQUIRE(num_pairs < (int64_t(1) << 29), "conv_pairs: too many pairs");
   const int64_t ld = round_up(num_targets, 4), n = ld * K;
-  SPIRA_HIP_REQUIRE(workspace && workspace_bytes >= static_cast<size_t>(n + 4 + 6 * num_pairs) * sizeof(int32_t),
-                    "conv_pairs: workspace too small (spira_hip_conv_compact_workspace)");
+  const int64_t nh = round_up(div_up(num_targets, compact::kTargets), 4);
+  // (16-byte parts: the rows and the blocks' heads, cleared together, the count
+  // of repeated pairs, the pairs)
+  SPIRA_HIP_REQUIRE(workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
+                        workspace_bytes >= static_cast<size_t>(n + nh + 4 + 8 * num_pairs) * sizeof(int32_t),
+                    "conv_pairs: workspace too small (spira_hip_conv_compact_workspace) or not 16-byte aligned");
   auto *idx = static_cast<int32_t *>(workspace);
-  int32_t *nextra = idx + n, *extra = nextra + 4;
-  hipLaunchKernelGGL(compact::rows_clear_kernel, dim3(div_up(std::max<int64_t>(n / 4, 1), 256)), dim3(256), 0, stream,
-                     idx, n / 4, nextra);
+  int32_t *heads = idx + n, *nextra = heads + nh;
+  auto *extra = reinterpret_cast<int4 *>(nextra + 4);
+  hipLaunchKernelGGL(compact::rows_clear_kernel, dim3(div_up((n + nh) / 4, 256)), dim3(256), 0, stream, idx,
+                     (n + nh) / 4, nextra);
   SPIRA_HIP_LAUNCH_CHECK();
   if (num_pairs > 0) {
     hipLaunchKernelGGL(compact::pair_rows_kernel, dim3(div_up(num_pairs, 256)), dim3(256), 0, stream, in_idx, out_idx,
-                       naddrs, rows, num_pairs, mirror_rows, num_sources, num_targets, ld, idx, extra,
-                       nextra);
+                       naddrs, rows, num_pairs, mirror_rows, num_sources, num_targets, ld, idx, heads, extra, nextra);
     SPIRA_HIP_LAUNCH_CHECK();
   }
   compact::Entries en{};
@@ -817,7 +836,7 @@ int spira_hip_conv_pairs(int64_t num_sources, int64_t num_targets, const int32_t
   en.dense = dense_map;
   en.kd = dense_offsets;
   en.extra = extra;
-  en.nextra = nextra;
+  en.heads = heads;
   return compact::launch(dtype, stream, en, num_targets, K + dense_offsets,
                          make_layer(sources, num_sources, row_channels, c_in, weights, fragments, c_out, dtype, targets,
                                     scale, shift, residual, relu));

@@ -14,9 +14,11 @@
 //   grid_count_kernel  set bits per block, kBlocks equal shares of a level;
 //   grid_emit_kernel   each block's keys after those of the blocks before.
 // Bound by the launches and, in wide scenes, by three passes over the words:
-// the words taken are at most kWordsPerKey per key (and kWordsLeast), so that
-// these passes stay below the searches that they replace.  A box with more
-// cells sets bit 1 of the flag and leaves the outputs undefined; the merging
+// the words taken are at most kWordsPerKey per key (and kWordsLeast: 64 MB; up
+// to kWordsMost: 256 MB), so that these passes stay below the searches that
+// they replace.  (A network's map build, us, by merging -> by grids: 100k
+// voxels of a sweep over 3200 x 3200 x 90 cells, 6.0M words, 285 -> 235, over
+// 4800 x 4800 x 90, 13.5M words, 285 -> 268.)  A box with more cells sets bit 1 of the flag and leaves the outputs undefined; the merging
 // chain (spira_hip_downsample_chain) is then the call.
 #include "common.hpp"
 #include "../../../include/spira_hip.h"
@@ -30,7 +32,7 @@ namespace grid {
 constexpr int kLevels = 8;
 constexpr int kBoxBlocks = 256;
 constexpr int kBlocks = 512;                            // blocks per level of the count and the emission
-constexpr int64_t kWordsPerKey = 32, kWordsLeast = int64_t(1) << 22, kWordsMost = int64_t(1) << 28;
+constexpr int64_t kWordsPerKey = 32, kWordsLeast = int64_t(1) << 24, kWordsMost = int64_t(1) << 26;
 constexpr uint32_t kUnsorted = 1, kTooWide = 2;
 
 struct Strides {

@@ -801,7 +801,11 @@ torch::Tensor forward_ws(int64_t S, int64_t T, int64_t gather_tile, int64_t scat
 // 50k pairs in all (20 -> 48, 24k pairs 18 -> 22, 90k 40 -> 32).  fp32's fused pass runs on the vector ALU: it wins only small
 // layers (100M multiply-adds at 27 offsets 40 -> 43, 245M 86 -> 59, 800M 535 ->
 // 70; with 125 offsets 120M 48 -> 76, 390M 214 -> 186).
+// Lists of more pairs than one per offset and target repeat some (points summed
+// into voxels): the compacted kernel adds repeats one by one (10 % of a list
+// 123 us, fused 85), the fused pass takes them as any other.
 static bool pairs_compact_pays(int64_t pairs, int64_t T, int64_t K, int64_t cin, int64_t cout, int dtype) {
+  if (pairs > T * K) return false;
   if (dtype == SPIRA_F32)
     return static_cast<double>(pairs) * cin * cout >= 1e8 * std::max(1.0, static_cast<double>(K) / 32);
   const double d = 64.0 * pairs / (static_cast<double>(std::max<int64_t>(T, 1)) * K);
@@ -1092,6 +1096,10 @@ void register_conv(pybind11::module_ &m) {
   m.def("cuda_time_gemm", &time_gemm);
   m.def("cuda_time_gather", &time_gather);
   m.def("cuda_time_scatter", &time_scatter);
+  // the side of pairs_compact_pays that a list falls on
+  m.def("pairs_compact_pays", [](int64_t pairs, int64_t T, int64_t K, const torch::Tensor &W) {
+    return pairs_compact_pays(pairs, T, K, W.size(1), W.size(2), dtype_of(W));
+  });
   m.def("cuda_free_buffers", &free_buffers);
   m.def("cuda_reset_error", &reset_error);
   m.def("set_os_row_order", &set_row_order);

@@ -14,6 +14,7 @@ import pytest
 import torch
 
 from spira_amd.nn import functional as F
+from spira_amd.nn.functional import _native
 
 from helpers import np_, rel_err
 
@@ -103,29 +104,37 @@ def _pair_list(lists, dev, unused=0):
     return [torch.from_numpy(np.ascontiguousarray(a)).to(dev) for a in (naddrs, qn, nb)]
 
 
-@pytest.mark.parametrize("repeat", [False, True])
+#                S     T    K  cin cout  compacted (fp16, fp32)
+PAIR_SHAPES = [(2100, 2000, 27, 64, 64, True, True), (2600, 2500, 8, 96, 100, True, True),
+               (900, 901, 40, 128, 64, True, True), (1500, 1400, 8, 96, 100, True, False),
+               (900, 901, 40, 128, 48, False, True)]
+
+
+@pytest.mark.parametrize("repeat", [0, 50, 1])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
-@pytest.mark.parametrize("S,T,K,cin,cout", [(2100, 2000, 27, 64, 64), (1500, 1400, 8, 96, 100), (900, 901, 40, 128, 48)])
-def test_pairs(dev, dtype, S, T, K, cin, cout, repeat):
-    """Dense enough for the compacted kernel; rows of pairs shuffled, and with
-    `repeat` every 50th pair given twice (both count)."""
+@pytest.mark.parametrize("S,T,K,cin,cout,half,full", PAIR_SHAPES)
+def test_pairs(dev, dtype, S, T, K, cin, cout, half, full, repeat):
+    """Lists on both sides of the compacted kernel's rule (repeats aside); rows
+    of pairs shuffled, and with `repeat` every so many-th pair given twice (both
+    count)."""
     lists = _lists(S, T, K, 0.6, S + K)
-    if repeat:
-        lists = [(np.concatenate([s, s[::50]]), np.concatenate([t, t[::50]])) for s, t in lists]
+    compacted = half if dtype == torch.float16 else full
     X, W, epi = _data(S, T, K, cin, cout, dtype, K)
-    sizes = np.array([len(s) for s, _ in lists])
-    naddrs = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
-    qn = np.concatenate([[0], np.cumsum((sizes + 127) // 128 * 128)]).astype(np.int32)
-    nb = np.stack([np.concatenate([s for s, _ in lists]), np.concatenate([t for _, t in lists])]).astype(np.int32)
-    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
-    y = F.sparse_convolution_forward_ws_merged(S, T, X.to(dev), W.to(dev), d(naddrs), d(qn), d(nb), nb.shape[1],
-                                               int(qn[-1]), epilogue=_dev(epi, dev))
+    pairs = sum(len(s) for s, _ in lists)
+    assert _native._C.pairs_compact_pays(pairs, T, K, W) == compacted
+    assert _native._C.pairs_compact_pays(pairs, S, K, W) == compacted
+    assert not _native._C.pairs_compact_pays(T * K + 1, T, K, W)  # (some must be repeated)
+    if repeat:
+        lists = [(np.concatenate([s, s[::repeat]]), np.concatenate([t, t[::repeat]])) for s, t in lists]
+    naddrs, qn, nb = _pair_list(lists, dev)
+    y = F.sparse_convolution_forward_ws_merged(S, T, X.to(dev), W.to(dev), naddrs, qn, nb, nb.shape[1], int(qn[-1]),
+                                               epilogue=_dev(epi, dev))
     assert rel_err(np_(y.float()), _ref(lists, T, X, W, epi)) <= TOL[dtype]
     # transposed: sources and targets exchanged
     back = [(t, s) for s, t in lists]
     X2, _, _ = _data(T, S, K, cin, cout, dtype, K + 1)
-    y = F.sparse_convolution_forward_ws_merged(T, S, X2.to(dev), W.to(dev), d(naddrs), d(qn), d(nb), nb.shape[1],
-                                               int(qn[-1]), True)
+    y = F.sparse_convolution_forward_ws_merged(T, S, X2.to(dev), W.to(dev), naddrs, qn, nb, nb.shape[1], int(qn[-1]),
+                                               True)
     assert rel_err(np_(y.float()), _ref(back, S, X2, W)) <= TOL[dtype]
 
 
@@ -156,6 +165,7 @@ def test_mirrored_pairs(dev, dtype, dense, repeat, unused):
     Kw = 27 if dense < 0 else 2 * rows
     full = kept + [(t, s) for s, t in kept[::-1]][Kw % 2:]
     X, W, epi = _data(S, T, Kw + Kos, cin, cout, dtype, 1)
+    assert bool(_native._C.pairs_compact_pays(nb.shape[1] * 2 - 2 * T, T, Kw + Kos, W))
     args = (X.to(dev), W.to(dev), naddrs, qn, nb)
     if dense < 0:
         y = F.sparse_convolution_forward_ws_merged(S, T, *args, nb.shape[1], int(qn[-1]), epilogue=_dev(epi, dev))
