@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from oracle import oracle as orc
+from spira_amd.nn import KernelMapCache
 from spira_amd.nn import functional as F
 
 from helpers import np_
@@ -32,6 +33,7 @@ SCENES = {
     "ends32": (np.array([[0, 4000, 200], [4095, 4095, 255], [4095, 4094, 255]], np.int32), False, S4[:1]),
     "eight": (_box(4000, (500, 500, 300), 6), True, [(2 ** l,) * 3 for l in range(1, 9)]),
     "nine": (_box(4000, (500, 500, 300), 6), True, [(2 ** l,) * 3 for l in range(1, 10)]),
+    "sweep": (_box(5000, (3200, 3200, 90), 9), True, S4),
     "too_wide": (_box(700, (60000, 60000, 4000), 7), True, S4),
 }
 
@@ -58,3 +60,21 @@ def test_unsorted_is_flagged(dev):
     assert F.downsample_chain_launch(k, S4, grid=True)[1].tolist()[-1] == 1
     for o, s in zip(F.streamed_output_generate(k, S4), S4):
         assert np.array_equal(np_(o), orc.downsample(keys, s)), s
+
+
+@pytest.mark.parametrize("name", ["words", "sweep", "too_wide"])
+def test_network_levels(dev, name):
+    """The levels that a network's map build takes, by grids or by merging; a
+    build after one that was too wide merges straight away, for a while."""
+    c, double, strides = SCENES[name]
+    keys, _ = orc.flatten_sort(c, double)
+    k = torch.from_numpy(keys).to(dev)
+    cache = KernelMapCache()
+    n = len(strides)
+    for i in range(3):
+        cache.reset()
+        cache.add_all_kernel_maps(k, [3] * (2 * n + 1), [(1, 1, 1)] * 2 + [s for s in strides for _ in range(2)],
+                                  strides, (1, 1, 1), [0] * (2 * n + 1))
+        for s in strides:
+            assert np.array_equal(np_(cache.get_target_coordinates(k, (1, 1, 1), s)), orc.downsample(keys, s)), s
+        assert cache._merge_builds == (max(0, cache.MERGE_BUILDS - i) if name == "too_wide" else 0)
