@@ -347,7 +347,9 @@ void prepare_row_orders(const std::vector<torch::Tensor> &maps, const std::vecto
     SPIRA_CHECK_ARG(map.size(0) >= Ts[i], "out_in_map has fewer rows than targets");
     SPIRA_CHECK_ARG(requests[i] >= -1 && requests[i] <= 1, "row order request must be -1, 0 or 1");
     const int64_t K = map.size(1);
-    const bool along = row_order_enabled() && requests[i] == -1 && K == 27 && Ts[i] >= kLeast && rows >= kTogether;
+    // (a map made under inference mode has no version to keep an order by)
+    const bool along = row_order_enabled() && requests[i] == -1 && K == 27 && Ts[i] >= kLeast &&
+                       rows >= kTogether && !map.is_inference();
     if ((!along && !row_order_applies(Ts[i], K, static_cast<int>(requests[i]))) || cached_order(map, Ts[i])) continue;
     bool dup = false;  // (one map listed twice)
     for (size_t j : batch) dup |= maps[j].unsafeGetTensorImpl() == map.unsafeGetTensorImpl();
