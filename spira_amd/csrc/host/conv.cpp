@@ -166,8 +166,8 @@ struct OrderEntry {
   const void *data = nullptr;
   uint32_t version = 0;
   int64_t T = 0;
-  bool free = false;  // made with the map at no sorting cost (convert_transposed_os_ordered)
-                      // or sorted along with a network's other maps (prepare_row_orders)
+  bool free = false;   // made with the map at no sorting cost (convert_transposed_os_ordered)
+  bool along = false;  // sorted along with a network's other maps (prepare_row_orders)
   torch::Tensor order, masks, ordered_map;
   hipStream_t stream = nullptr;  // the stream the tensors were allocated and written on
 };
@@ -361,7 +361,9 @@ void prepare_row_orders(const std::vector<torch::Tensor> &maps, const std::vecto
   for (size_t b0 = 0; b0 < batch.size(); b0 += 16) {
     const size_t nb = std::min<size_t>(16, batch.size() - b0);
     if (nb == 1) {
-      row_order_of(maps[batch[b0]], Ts[batch[b0]]);
+      const torch::Tensor &map = maps[batch[b0]];
+      row_order_of(map, Ts[batch[b0]]);
+      order_cache().find(map.unsafeGetTensorImpl())->second.along = requests[batch[b0]] == -1;
       continue;
     }
     purge_expired_orders();
@@ -376,7 +378,7 @@ void prepare_row_orders(const std::vector<torch::Tensor> &maps, const std::vecto
       e.version = map._version();
       e.T = T;
       e.stream = current_stream();
-      e.free = requests[batch[b0 + q]] == -1;
+      e.along = requests[batch[b0 + q]] == -1;
       e.order = empty_i32({T}, map.device());
       e.masks = torch::empty({(T + 127) / 128 * 2}, torch::TensorOptions(map.device()).dtype(torch::kInt64));
       e.ordered_map = empty_i32({T, K}, map.device());
@@ -561,7 +563,7 @@ static void run_os(const torch::Tensor *map, int64_t S, int64_t T, const torch::
     if (row_order_applies(T, K, tn.row_order)) oe = &row_order_of(*map, T);
     else if (tn.row_order != 0 && row_order_enabled()) {
       oe = cached_order(*map, T);
-      if (oe && !oe->free) oe = nullptr;  // (a sorted order only by the rule or on request)
+      if (oe && !oe->free && !oe->along) oe = nullptr;  // (a sorted order only by the rules or on request)
     }
     if (oe) {
       record_use(oe->stream, {&oe->order, &oe->masks, &oe->ordered_map});
@@ -1106,9 +1108,14 @@ void register_conv(pybind11::module_ &m) {
   m.def("cuda_reset_error", &reset_error);
   m.def("set_os_row_order", &set_row_order);
   m.def("kmap_row_order", &kmap_row_order);
-  // an order made with the map (no sort), as a partition inverse carries one
   // number of cached row orders (for tests: entries of freed maps are dropped)
   m.def("row_order_cache_size", [] { return static_cast<int64_t>(order_cache().size()); });
+  // whether an fp16 layer with no request of its own walks `map` in an order that it finds cached
+  m.def("finds_row_order", [](const torch::Tensor &map, int64_t T) {
+    const OrderEntry *e = cached_order(map, T);
+    return e != nullptr && (e->free || e->along || row_order_applies(T, map.size(1)));
+  });
+  // an order made with the map (no sort), as a partition inverse carries one
   m.def("has_free_row_order", [](const torch::Tensor &map, int64_t T) {
     const OrderEntry *e = cached_order(map, T);
     return e != nullptr && e->free;

@@ -1,9 +1,10 @@
-"""Which maps of a network are put in row order with its map build: what the
-layers then find, for maps without a version (inference tensors)."""
+"""Which maps of a network are put in row order with its map build, and what its
+layers then find."""
 import pytest
 import torch
 
 from spira_amd.nn import functional as F
+from spira_amd.nn.functional import _native
 
 from helpers import np_, rel_err
 
@@ -36,3 +37,15 @@ def test_maps_of_inference_mode(dev):
                 y = F.sparse_convolution_forward_os(1000, T, a, X, W)
                 y0 = F.sparse_convolution_forward_os(1000, T, b, X, W, tuning=(0, 0, 0, 0, 0, 0))
                 assert rel_err(np_(y.float()), np_(y0.float())) <= (4e-3 if dtype == torch.float16 else 1e-5)
+
+
+def test_one_map_left_over(dev):
+    """17 maps, sorted as 16 and one: layers find every order, and none counts
+    as free of the sort."""
+    sizes = (12000,) * 17
+    maps = _maps(dev, sizes, 1)
+    F.prepare_row_orders(maps, list(sizes), [-1] * 17)
+    for m, T in zip(maps, sizes):
+        assert _native._C.finds_row_order(m, T) and not _native._C.has_free_row_order(m, T)
+    other = _maps(dev, (12000,), 2)[0]
+    assert not _native._C.finds_row_order(other, 12000)
