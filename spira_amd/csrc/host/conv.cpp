@@ -1110,6 +1110,8 @@ void register_conv(pybind11::module_ &m) {
   m.def("kmap_row_order", &kmap_row_order);
   // number of cached row orders (for tests: entries of freed maps are dropped)
   m.def("row_order_cache_size", [] { return static_cast<int64_t>(order_cache().size()); });
+  m.def("cached_row_order",
+        [](const torch::Tensor &map, int64_t T) { return cached_order(map, T) != nullptr; });
   // whether an fp16 layer with no request of its own walks `map` in an order that it finds cached
   m.def("finds_row_order", [](const torch::Tensor &map, int64_t T) {
     const OrderEntry *e = cached_order(map, T);

@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import contextlib
 import operator
+import weakref
 from typing import Any, Dict, List, Optional, Tuple, Union
 
 import numpy as np
@@ -36,8 +37,8 @@ class KernelMapCache:
     ``(source stride, target stride, kernel size)``."""
 
     #: queue the row orders of the large output-stationary maps with the
-    #: network-wide map build (only the fp16 convolution kernel uses them; a
-    #: network run in fp32 can turn this off to skip that work)
+    #: network-wide map build.  Only the fp16 convolution kernel uses them: a
+    #: cache attached to layers none of which is in fp16 makes none.
     prepare_row_orders = True
 
     #: builds that merge their levels straight away after one whose voxels lay
@@ -55,6 +56,19 @@ class KernelMapCache:
         #: entry follow the library's default rule.  Set by the selector.
         self.row_order_requests: Dict[tuple, int] = {}
         self._merge_builds = 0
+        self._layers = weakref.WeakSet()  # the layers it is attached to (set_kernel_map_cache)
+
+    def __getstate__(self):
+        # (weak references are neither copied nor pickled: a copy knows no layers)
+        return {k: v for k, v in self.__dict__.items() if k != "_layers"}
+
+    def __setstate__(self, state) -> None:
+        self.__init__()
+        self.__dict__.update(state)
+
+    def _orders_read(self) -> bool:
+        """A layer may walk its maps in row order (also where none has said)."""
+        return not self._layers or any(m.kernel.dtype == torch.float16 for m in self._layers)
 
     def reset(self) -> None:
         self._coordinates_cache.clear()
@@ -162,7 +176,7 @@ class KernelMapCache:
         kmaps += F.build_kmap_streamed(voxels, kernel_sizes, src_strides, dataflow, begin=first)
         # the row orders of the large output-stationary maps, all in one
         # batched chain of launches
-        if self.prepare_row_orders:
+        if self.prepare_row_orders and self._orders_read():
             sel = [i for i in range(len(kernel_sizes)) if dataflow[i] == 0]
             if sel:
                 F.prepare_row_orders([kmaps[i][2] for i in sel], [kmaps[i][1] for i in sel],
@@ -236,7 +250,11 @@ class SparseConv(Module):
                 self.bias.uniform_(-bound, bound)
 
     def set_kernel_map_cache(self, cache: KernelMapCache) -> None:
+        if self._kernel_map_cache is not None:
+            self._kernel_map_cache._layers.discard(self)
         self._kernel_map_cache = cache
+        if cache is not None:
+            cache._layers.add(self)
 
     @property
     def is_trivial(self) -> bool:

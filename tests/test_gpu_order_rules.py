@@ -1,8 +1,15 @@
 """Which maps of a network are put in row order with its map build, and what its
 layers then find."""
+import copy
+import gc
+import pickle
+
 import pytest
 import torch
 
+from spira_amd import nn as spnn
+from spira_amd import scenes
+from spira_amd.networks import kmap_schedule
 from spira_amd.nn import functional as F
 from spira_amd.nn.functional import _native
 
@@ -49,3 +56,37 @@ def test_one_map_left_over(dev):
         assert _native._C.finds_row_order(m, T) and not _native._C.has_free_row_order(m, T)
     other = _maps(dev, (12000,), 2)[0]
     assert not _native._C.finds_row_order(other, 12000)
+
+
+def test_only_for_layers_that_read_them(dev):
+    """A network's map build orders maps of a cache attached to an fp16 layer, or
+    to none that it knows of; not those of a network in float32, nor its copy's."""
+    coords = scenes.indoor(target=120_000, seed=3)
+    keys, _ = F.flat_sort(torch.from_numpy(coords).to(dev), True)
+    ts, ks, ss = kmap_schedule("UNet")
+
+    def build(cache):
+        """(27-offset maps in row order, their rows) of a build."""
+        cache.reset()
+        cache.add_all_kernel_maps(keys, ks, ss, ts, (1, 1, 1), [0] * len(ks))
+        maps = [e for key, e in cache._kernel_maps_cache.items() if key[2] == (3, 3, 3)]
+        return sum(_native._C.cached_row_order(e[3], e[2]) for e in maps)
+
+    cache = spnn.KernelMapCache()
+    orders = build(cache)
+    assert orders >= 2
+    a, b = spnn.SparseConv(4, 8, 3).to(dev), spnn.SparseConv(8, 8, 3).to(dev)
+    a.set_kernel_map_cache(cache)
+    b.set_kernel_map_cache(cache)
+    assert build(cache) == 0
+    a.half()
+    assert build(cache) == orders
+    other = spnn.KernelMapCache()
+    a.set_kernel_map_cache(other)
+    assert build(cache) == 0 and build(other) == orders
+    twin = copy.deepcopy(b)
+    assert twin._kernel_map_cache is not cache and build(twin._kernel_map_cache) == orders
+    assert build(pickle.loads(pickle.dumps(spnn.KernelMapCache()))) == orders
+    del b
+    gc.collect()
+    assert build(cache) == orders  # (attached to none again)
