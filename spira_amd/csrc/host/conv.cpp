@@ -142,9 +142,9 @@ static torch::Tensor compact_rows(const torch::Tensor &X) {
 
 // The compacted kernels address the source rows and an offset's weights with
 // 31-bit byte offsets.
-static bool compact_fits(const torch::Tensor &X, const torch::Tensor &W) {
-  const int64_t v = 16 / X.element_size();
-  return X.size(0) * ((X.size(1) + v - 1) / v * 16) < (int64_t(1) << 31) &&
+static bool compact_fits(int64_t rows, const torch::Tensor &W) {
+  const int64_t v = 16 / W.element_size();
+  return rows * ((W.size(1) + v - 1) / v * 16) < (int64_t(1) << 31) &&
          (W.size(1) + 64) * W.size(2) * 4 < (int64_t(1) << 31);
 }
 
@@ -539,7 +539,7 @@ static void run_os(const torch::Tensor *map, int64_t S, int64_t T, const torch::
   // pad first (a launch of its own: 3 -> 32 channels down-sampling 5k voxels
   // 12 -> 16 us; 20k targets x 8 offsets and more are faster with it)
   const bool small_unaligned = X.size(1) % 4 != 0 && T * K < 200000;
-  if (dtype == SPIRA_F32 && mp && mode == SPIRA_OUT_STORE && T > 0 && !small_unaligned && compact_fits(X, W)) {
+  if (dtype == SPIRA_F32 && mp && mode == SPIRA_OUT_STORE && T > 0 && !small_unaligned && compact_fits(X.size(0), W)) {
     auto Xr = compact_rows(X);
     check_rc(spira_hip_conv_map(X.size(0), T, K, mp, Xr.data_ptr(), Xr.size(1), W.size(1), wrow_ptr(W, w0),
                                 nullptr, W.size(2), dtype, out, epi.scale, epi.shift, epi.residual, epi.relu,
@@ -708,7 +708,7 @@ static bool masks_compact(int64_t S, int64_t T, const torch::Tensor &X, const to
                           const torch::Tensor &source_masks, const torch::Tensor &target_masks,
                           const torch::Tensor &nbsizes, bool half, const torch::Tensor *dense, int Kos, const Epi &e,
                           torch::Tensor &Y) {
-  if (!compact_fits(X, W) || W.numel() == 0) return false;
+  if (!compact_fits(X.size(0), W) || W.numel() == 0) return false;
   check_masks(S, T, source_masks, target_masks);
   const int Km = static_cast<int>(target_masks.size(0));
   const int nh = half ? (Km + 1) / 2 : Km;
@@ -766,6 +766,26 @@ static void gs_scatter(GsPlan &p, int cout, int dtype, const float *base, void *
            "scatter");
 }
 
+// The buffered phases (dense: a hybrid's first offsets, or null with Kos 1 for
+// the identity; Kos 0: none).
+static torch::Tensor ws_buffered(int64_t S, int64_t T, const std::optional<double> &threshold, const torch::Tensor &X,
+                                 const torch::Tensor &W, const torch::Tensor &source_masks,
+                                 const torch::Tensor &target_masks, const torch::Tensor &nbsizes, bool half,
+                                 const torch::Tensor *dense, int Kos, const Epi &e) {
+  torch::Tensor acc;
+  if (Kos > 0) {
+    acc = torch::empty({T, W.size(2)}, X.options().dtype(torch::kFloat));
+    run_os(dense, S, T, X, W, 0, Kos, acc.data_ptr<float>(), SPIRA_OUT_STORE_F32);
+  }
+  auto Y = torch::empty({T, W.size(2)}, X.options());
+  auto s = current_stream();
+  auto p = plan_gs(S, T, source_masks, target_masks, nbsizes, half, threshold, W.size(1), W.size(2), X.options());
+  gs_gather(p, X, s);
+  gs_gemm(p, W, Kos, s);
+  gs_scatter(p, W.size(2), dtype_of(X), acc.defined() ? acc.data_ptr<float>() : nullptr, Y.data_ptr(), s, e);
+  return Y;
+}
+
 // (reference: CUDASparseConvolutionForward_WS, :130-184)
 torch::Tensor forward_ws(int64_t S, int64_t T, int64_t gather_tile, int64_t scatter_tile, int64_t parallel,
                          const std::optional<double> &threshold, const torch::Tensor &X, const torch::Tensor &W,
@@ -782,14 +802,9 @@ torch::Tensor forward_ws(int64_t S, int64_t T, int64_t gather_tile, int64_t scat
   const int Km = static_cast<int>(target_masks.size(0));
   const bool half = (Km % 2 == 1) && S == T;
   auto Y = torch::empty({T, W.size(2)}, X.options());
-  auto s = current_stream();
   const Epi e = epi_of(scale, shift, residual, relu, T, W.size(2), X);
   if (masks_compact(S, T, X, W, source_masks, target_masks, nbsizes, half, nullptr, 0, e, Y)) return Y;
-  auto p = plan_gs(S, T, source_masks, target_masks, nbsizes, half, threshold, W.size(1), W.size(2), X.options());
-  gs_gather(p, X, s);
-  gs_gemm(p, W, 0, s);
-  gs_scatter(p, W.size(2), dtype_of(X), nullptr, Y.data_ptr(), s, e);
-  return Y;
+  return ws_buffered(S, T, threshold, X, W, source_masks, target_masks, nbsizes, half, nullptr, 0, e);
 }
 
 // Whether a pair list goes to the compacted kernel or to the fused pass with
@@ -839,7 +854,7 @@ static std::optional<torch::Tensor> pairs_compact(int64_t S, int64_t T, const to
                           int64_t mapsize, bool transpose, int mirror_rows, const torch::Tensor *dense, int Kos,
                           const Epi &e) {
   const int rows = static_cast<int>(naddrs.size(0) - 1);
-  if (!compact_fits(X, W) || W.numel() == 0 || mapsize >= (int64_t(1) << 29)) return std::nullopt;
+  if (!compact_fits(X.size(0), W) || W.numel() == 0 || mapsize >= (int64_t(1) << 29)) return std::nullopt;
   // (about T pairs in a self-mirrored centre row, taken once, and in a
   // hybrid's dense offsets)
   const int64_t pairs = (mirror_rows > 0 ? 2 : 1) * mapsize - (mirror_rows % 2 == 1 ? T : 0) + (Kos > 0 ? T : 0);
@@ -925,17 +940,27 @@ torch::Tensor forward_hs(int64_t S, int64_t T, int64_t gather_tile, int64_t scat
   SPIRA_CHECK_ARG(W.size(0) == Kws + Kos, "weights have ", W.size(0), " offsets, expected ", Kws + Kos);
   const torch::Tensor *dense = out_in_map.has_value() ? &*out_in_map : nullptr;
   auto Y = torch::empty({T, W.size(2)}, X.options());
-  auto s = current_stream();
   const Epi e = epi_of(scale, shift, residual, relu, T, W.size(2), X);
   check_dense(dense, S, T, Kos);
   if (masks_compact(S, T, X, W, source_masks, target_masks, nbsizes, true, dense, Kos, e, Y)) return Y;
-  auto acc = torch::empty({T, W.size(2)}, X.options().dtype(torch::kFloat));
-  run_os(dense, S, T, X, W, 0, Kos, acc.data_ptr<float>(), SPIRA_OUT_STORE_F32);
-  auto p = plan_gs(S, T, source_masks, target_masks, nbsizes, true, threshold, W.size(1), W.size(2), X.options());
-  gs_gather(p, X, s);
-  gs_gemm(p, W, Kos, s);
-  gs_scatter(p, W.size(2), dtype_of(X), acc.data_ptr<float>(), Y.data_ptr(), s, e);
-  return Y;
+  return ws_buffered(S, T, threshold, X, W, source_masks, target_masks, nbsizes, true, dense, Kos, e);
+}
+
+// The buffered phases of forward_ws (hybrid false) and forward_hs, which layers
+// take whose features are too large for the compacted kernel.  No reference
+// counterpart: it lets a test see them on small ones.
+torch::Tensor forward_buffered(int64_t S, int64_t T, const std::optional<double> &threshold, const torch::Tensor &X,
+                               const torch::Tensor &W, const torch::Tensor &source_masks,
+                               const torch::Tensor &target_masks, const torch::Tensor &nbsizes, bool hybrid,
+                               const std::optional<torch::Tensor> &out_in_map) {
+  check_features(X, W);
+  const int Km = static_cast<int>(target_masks.size(0));
+  const torch::Tensor *dense = out_in_map.has_value() ? &*out_in_map : nullptr;
+  const int Kos = !hybrid ? 0 : dense ? static_cast<int>(dense->size(1)) : 1;
+  SPIRA_CHECK_ARG(W.size(0) == Km + Kos, "weights have ", W.size(0), " offsets, expected ", Km + Kos);
+  if (hybrid) check_dense(dense, S, T, Kos);
+  return ws_buffered(S, T, threshold, X, W, source_masks, target_masks, nbsizes, hybrid || (Km % 2 == 1 && S == T),
+                     dense, Kos, Epi());
 }
 
 // (reference: CUDASparseConvolutionForward_HS_Merged, :346-443)
@@ -1100,6 +1125,11 @@ void register_conv(pybind11::module_ &m) {
   m.def("cuda_time_gemm", &time_gemm);
   m.def("cuda_time_gather", &time_gather);
   m.def("cuda_time_scatter", &time_scatter);
+  m.def("forward_buffered", &forward_buffered, py::arg("S"), py::arg("T"), py::arg("threshold"), py::arg("X"),
+        py::arg("W"), py::arg("source_masks"), py::arg("target_masks"), py::arg("nbsizes"), py::arg("hybrid") = false,
+        py::arg("out_in_map") = py::none());
+  // whether a mask layer of S sources and weights W takes the compacted kernel
+  m.def("masks_compact", [](int64_t S, const torch::Tensor &W) { return compact_fits(S, W) && W.numel() > 0; });
   // the side of pairs_compact_pays that a list falls on
   m.def("pairs_compact_pays", [](int64_t pairs, int64_t T, int64_t K, const torch::Tensor &W) {
     return pairs_compact_pays(pairs, T, K, W.size(1), W.size(2), dtype_of(W));

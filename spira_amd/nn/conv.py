@@ -264,7 +264,8 @@ class SparseConv(Module):
     def tune_gs(self, free_buffers: bool = True):
         """Record (masks, sizes) of gather-scatter runs while inside, then sweep
         the bucket threshold by timing the grouped GEMM (reference
-        conv.py:217-307).  The reference's gather / scatter tile sweep has no
+        conv.py:217-307), over the runs that have buckets: those whose features
+        are too large for the compacted kernel.  The reference's gather / scatter tile sweep has no
         counterpart here: the gather and scatter kernels of this build have
         no tile parameter (the keys stay in the config for file
         compatibility); the CDNA4 launch choices are swept by ``tune_os``."""
@@ -275,14 +276,16 @@ class SparseConv(Module):
             yield
             if free_buffers:
                 F.cuda_free_buffers()
-            if self.is_trivial or not self._tuning_data:
+            from .functional import _native
+            data = [d for d in self._tuning_data if not _native._C.masks_compact(d[0].shape[1], self.kernel)]
+            if self.is_trivial or not data:
                 return
             best = None
             for thr in self.__AVAILABLE_THRESHOLD__:
                 try:
                     t = [F.cuda_time_gemm(threshold=thr, weights=self.kernel, source_masks=sm, target_masks=tm,
                                           kernel_map_sizes=nb)
-                         for _ in range(self.__NUM_TUNING_ROUNDS__) for sm, tm, nb in self._tuning_data]
+                         for _ in range(self.__NUM_TUNING_ROUNDS__) for sm, tm, nb in data]
                 except RuntimeError:
                     F.cuda_reset_error()
                     break

@@ -9,6 +9,7 @@ import torch
 from oracle import oracle as orc
 from spira_amd import scenes
 from spira_amd.nn import functional as F
+from spira_amd.nn.functional import _native
 
 from helpers import np_, rel_err
 
@@ -77,6 +78,25 @@ def test_ws_gather_scatter_submanifold(dev, keys, dtype, threshold):
     y = F.sparse_convolution_forward_ws(S, T, X, W, _t(m[3], dev), _t(m[4], dev), _t(m[5], dev), 16, 16, None,
                                         threshold)
     ref = orc.conv_ws_gs(S, T, Xn, Wn, m[3], m[4])
+    assert rel_err(np_(y.float()), ref) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("threshold", [-1, 0.25, 0.5, 2.0, None])
+@pytest.mark.parametrize("dataflow,cin,cout", [(2, 64, 64), (2, 20, 36), (4, 32, 48), (6, 32, 32)])
+def test_buffered_phases(dev, keys, dtype, threshold, dataflow, cin, cout):
+    """Gather, grouped GEMM and scatter through their buffers (layers with
+    features too large for the compacted kernel) under every bucketing."""
+    m = orc.build_kmap(keys, keys, (3, 3, 3), (1, 1, 1), dataflow)
+    S = T = len(keys)
+    X, W, Xn, Wn = _data(S, 27, cin, cout, dtype, dev, seed=6)
+    dense = 0 if dataflow == 2 else int(orc.indexes_l1((3, 3, 3), dataflow)[0][0])
+    Y = None
+    if dense:
+        Y = orc.conv_os(m[2] if dataflow == 6 else np.arange(T, dtype=np.int32).reshape(T, 1), T, Xn, Wn[:dense])
+    ref = orc.conv_ws_gs(S, T, Xn, Wn, m[3], m[4], woffset=dense, Y=Y)
+    y = _native._C.forward_buffered(S, T, threshold, X, W, _t(m[3], dev), _t(m[4], dev), _t(m[5], dev), dense > 0,
+                                    _t(m[2], dev) if dataflow == 6 else None)
     assert rel_err(np_(y.float()), ref) <= TOL[dtype]
 
 

@@ -205,3 +205,23 @@ def test_os_tuning_keeps_results(dev, tmp_path):
     for a, b in zip(before, after):
         rms = float(a.pow(2).mean().sqrt()) or 1.0
         assert float((a - b).abs().max()) / rms <= 1e-2
+
+
+def test_threshold_sweep_only_where_it_matters(monkeypatch):
+    """The bucket threshold is timed for recorded runs whose features are too
+    large for the compacted kernel (here 2^26 rows of 32 float32 channels), and
+    left alone for the others."""
+    from spira_amd.nn import conv as conv_module
+    timed = []
+    monkeypatch.setattr(conv_module.F, "cuda_free_buffers", lambda: None)
+    monkeypatch.setattr(conv_module.F, "cuda_time_gemm",
+                        lambda threshold, **kw: timed.append(kw["source_masks"].shape) or (1.0 if threshold == 2.0 else 2.0))
+    conv = spira_amd.nn.SparseConv(32, 32, 3)
+    one = torch.zeros(27, 1, dtype=torch.int32)
+    for rows, threshold in ((1000, -1), (1 << 26, 2.0)):
+        timed.clear()
+        with conv.tune_gs():
+            conv._tuning_data.append((one.expand(27, rows), one, one[:, 0]))
+            conv._tuning_data.append((one.expand(27, 500), one, one[:, 0]))
+        assert conv.tunable_config["threshold"] == threshold
+        assert set(timed) == (set() if rows == 1000 else {(27, rows)})
