@@ -63,7 +63,7 @@ class KernelMapCache:
         return {k: v for k, v in self.__dict__.items() if k != "_layers"}
 
     def __setstate__(self, state) -> None:
-        self.__init__()
+        self.__dict__.update(_merge_builds=0, _layers=weakref.WeakSet())
         self.__dict__.update(state)
 
     def _orders_read(self) -> bool:
@@ -250,11 +250,10 @@ class SparseConv(Module):
                 self.bias.uniform_(-bound, bound)
 
     def set_kernel_map_cache(self, cache: KernelMapCache) -> None:
-        if self._kernel_map_cache is not None:
-            self._kernel_map_cache._layers.discard(self)
+        # (a cache of another class than KernelMapCache may keep no layers)
+        getattr(self._kernel_map_cache, "_layers", set()).discard(self)
         self._kernel_map_cache = cache
-        if cache is not None:
-            cache._layers.add(self)
+        getattr(cache, "_layers", set()).add(self)
 
     @property
     def is_trivial(self) -> bool:
