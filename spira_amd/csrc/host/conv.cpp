@@ -536,10 +536,15 @@ static void run_os(const torch::Tensor *map, int64_t S, int64_t T, const torch::
   check_dense(map, S, T, K);
   const int32_t *mp = map ? map->data_ptr<int32_t>() : nullptr;
   // fp32: the compacted kernel, but for small maps of rows it would have to
-  // pad first (a launch of its own: 3 -> 32 channels down-sampling 5k voxels
-  // 12 -> 16 us; 20k targets x 8 offsets and more are faster with it)
-  const bool small_unaligned = X.size(1) % 4 != 0 && T * K < 200000;
-  if (dtype == SPIRA_F32 && mp && mode == SPIRA_OUT_STORE && T > 0 && !small_unaligned && compact_fits(X.size(0), W)) {
+  // pad first (a launch of its own: 3 -> 32 channels down-sampling 60k voxels to
+  // 16k 12.0 -> 15.4 us; 20k targets x 8 offsets and more are mostly faster with
+  // it), and for narrow layers down-sampling a small solid scene, whose offsets
+  // nearly all hold a voxel (three sources per target and more: 50k to 14k
+  // voxels, 32 -> 32 12.1 -> 14.3; 2.7 sources per target 12.2 -> 12.8, 2.4 12.1
+  // -> 11.9; 3.0 and 33k targets 18.9 -> 16.3; 32 -> 48 17.4 -> 13.7)
+  const bool solid = K <= 8 && X.size(0) >= 3 * T && X.size(1) <= 32 && W.size(2) <= 32;
+  const bool small = T * K < 200000 && (X.size(1) % 4 != 0 || solid);
+  if (dtype == SPIRA_F32 && mp && mode == SPIRA_OUT_STORE && T > 0 && !small && compact_fits(X.size(0), W)) {
     auto Xr = compact_rows(X);
     check_rc(spira_hip_conv_map(X.size(0), T, K, mp, Xr.data_ptr(), Xr.size(1), W.size(1), wrow_ptr(W, w0),
                                 nullptr, W.size(2), dtype, out, epi.scale, epi.shift, epi.residual, epi.relu,

@@ -90,6 +90,20 @@ def test_fp32_map(dev, S, T, K, cin, cout, density):
     assert rel_err(np_(y), _ref(lists, T, X, W, epi)) <= TOL[torch.float32]
 
 
+@pytest.mark.parametrize("S,T,K,cin,cout", [(2999, 1000, 8, 32, 32), (3000, 1000, 8, 32, 32), (3000, 1000, 9, 32, 32),
+                                            (3000, 1000, 8, 36, 32), (3000, 1000, 8, 32, 33), (3000, 1000, 8, 5, 7),
+                                            (75000, 24999, 8, 16, 20), (75000, 25000, 8, 16, 20)])
+def test_fp32_map_of_a_solid_scene(dev, S, T, K, cin, cout):
+    """Nearly full maps of three sources per target: both sides of each line of
+    the rule that keeps narrow layers on small ones from the compacted kernel."""
+    m = np.random.default_rng(K).integers(-S // 15, S, (T, K)).clip(-1).astype(np.int32)
+    lists = [(m[m[:, k] >= 0, k], np.nonzero(m[:, k] >= 0)[0]) for k in range(K)]
+    X, W, epi = _data(S, T, K, cin, cout, torch.float32, K)
+    dm = torch.nn.functional.pad(torch.from_numpy(m), (0, 0, 0, -T % 128), value=-1).to(dev)
+    y = F.sparse_convolution_forward_os(S, T, dm, X.to(dev), W.to(dev), epilogue=_dev(epi, dev))
+    assert rel_err(np_(y), _ref(lists, T, X, W, epi)) <= TOL[torch.float32]
+
+
 def _pair_list(lists, dev, unused=0):
     """(naddrs, qnaddrs, nbmaps) on the device; with `unused` every 40th entry
     -1 on one side and that many entries past the last row's."""
