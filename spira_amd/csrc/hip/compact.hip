@@ -591,7 +591,7 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(const FT *__restrict__ X,
 // 68k-voxel level with 9.6 pairs per target 51 -> 70 us).  Two ring stages up
 // to 64 columns (three: 32 -> 32 24.6 -> 30.1 us, 64 -> 64 the same), three
 // beyond.  fp32 layers wider than 64 columns take several 64-column blocks
-// (128 -> 128, 20k voxels: 159 us with eight waves, 124 us).  16-column layers
+// (128 -> 128, 20k voxels: 121 us with eight waves, 96 us; 60k 413 and 415).  16-column layers
 // of more than 32 offsets take two waves, the second for the index lists
 // (125 offsets, 5k voxels: 66 us with one wave, 45 us).
 template <class FT, int PITCH, int NF>
@@ -619,7 +619,7 @@ static void launch_n(hipStream_t s, const Entries &en, int64_t T, int K, const L
 
 static int launch(int dtype, hipStream_t s, const Entries &en, int64_t T, int K, const Layer &l) {
   // fragments per step: the largest of 4, 3, 2 and 1 that divides a row's
-  // (fp32 64 -> 64 on 20k voxels: two per step 51 us, four 43 us)
+  // (fp32 64 -> 64 on 20k voxels: two per step 48 us, four 40 us)
   const bool f16 = dtype == SPIRA_F16;
   if (l.nft % 4 == 0) {
     if (f16) launch_n<_Float16, 256, 4>(s, en, T, K, l);

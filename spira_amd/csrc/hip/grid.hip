@@ -18,8 +18,9 @@
 // to kWordsMost: 256 MB), so that these passes stay below the searches that
 // they replace.  (A network's map build, us, by merging -> by grids: 100k
 // voxels of a sweep over 3200 x 3200 x 90 cells, 6.0M words, 299 -> 239, over
-// 4800 x 4800 x 90, 13.5M words, 295 -> 265.)  A box with more cells sets bit 1 of the flag and leaves the outputs undefined; the merging
-// chain (spira_hip_downsample_chain) is then the call.
+// 4800 x 4800 x 90, 13.5M words, 295 -> 265.)  A box with more cells sets bit 1
+// of the flag and leaves the outputs undefined; the merging chain
+// (spira_hip_downsample_chain) is then the call.
 #include "common.hpp"
 #include "../../../include/spira_hip.h"
 

@@ -822,9 +822,10 @@ torch::Tensor forward_ws(int64_t S, int64_t T, int64_t gather_tile, int64_t scat
 // 24 -> 34).  Columns that the compacted kernel pads (48 to 64, 96 of wide
 // inputs to 128) want more pairs (96 -> 48 at d = 5 48 -> 60, 96 -> 96 80 ->
 // 89, at 12 142 -> 115; 125 offsets 32 -> 48 75 -> 93), and channels that need padded rows, a launch more,
-// 50k pairs in all (20 -> 48, 24k pairs 18 -> 22, 90k 40 -> 32).  fp32's fused pass runs on the vector ALU: it wins only small
-// layers (100M multiply-adds at 27 offsets 40 -> 43, 245M 86 -> 59, 800M 535 ->
-// 70; with 125 offsets 120M 48 -> 76, 390M 214 -> 186).
+// 50k pairs in all (20 -> 48, 24k pairs 18 -> 22, 90k 40 -> 32).  fp32's fused
+// pass runs on the vector ALU: it wins only small layers (27 offsets: 46M
+// multiply-adds 22 -> 32, 113M 51 -> 36, 184M 57 -> 53, 450M 164 -> 48; 125
+// offsets: 99M 38 -> 109, 370M 210 -> 118, 397M of 128 channels 223 -> 196).
 // Lists of more pairs than one per offset and target repeat some (points summed
 // into voxels): the compacted kernel adds repeats one by one (10 % of a list
 // 123 us, fused 85), the fused pass takes them as any other.
